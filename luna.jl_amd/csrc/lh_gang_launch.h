@@ -1,0 +1,80 @@
+// lh_gang_launch.h -- launches of the gang kernels (lh_gang.h) and the memory
+// they need.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <string.h>
+
+#include "../../include/luna_hip.h"
+
+struct DInst;
+
+static constexpr int LG_G = 4;               // members of a gang
+static constexpr int LG_TWN = 32768;         // twiddle table: exp(-2πi m/LG_TWN)
+static constexpr int LG_MIN_WG = 32;         // workgroups of the smallest launch
+static constexpr int LG_XCC = 16;            // values of HW_REG_XCC_ID
+static constexpr int LG_FLAG_STRIDE = 32;    // unsigneds between two members' flags (one cache line)
+static constexpr int LG_SLOTS = 14;          // vectors of an instance's work block, see LgVec
+
+// Control block of one launch.
+struct GangCtl {
+    unsigned next_job, njobs, n_wg, left;
+    unsigned pad[12];
+    unsigned ticket[LG_XCC];
+    // then per job LG_G flags (LG_FLAG_STRIDE apart), then mail[LG_XCC][n_wg / LG_G] (64-bit)
+};
+__host__ __device__ constexpr size_t lg_flags_off() { return sizeof(GangCtl); }
+__host__ __device__ constexpr size_t lg_mail_off(size_t njobs) {
+    return sizeof(GangCtl) + njobs * LG_G * LG_FLAG_STRIDE * sizeof(unsigned);
+}
+__host__ __device__ constexpr size_t lg_ctl_bytes(size_t njobs, size_t n_wg) {
+    return lg_mail_off(njobs) + LG_XCC * (n_wg / LG_G) * sizeof(unsigned long long);
+}
+
+// Complex points of a transform and the work block of a mode-averaged class.
+static inline int lg_points(const lh_desc& d) { return d.grid_kind == LH_GRID_REAL ? d.n_to / 2 : d.n_to; }
+static inline size_t lg_stride(const lh_desc& d) {  // one vector of the work block
+    const int M = lg_points(d);
+    return (size_t)LG_G * ((d.grid_kind == LH_GRID_REAL ? M / 8 : M / 4) + 8);
+}
+static inline size_t lg_exchange_len(const lh_desc& d) {  // one exchange series
+    return (size_t)lg_points(d) * ((d.grid_kind == LH_GRID_REAL && d.raman) ? 2 : 1);
+}
+static inline size_t lg_area_len(const lh_desc& d) {  // complex points of the exchange area
+    return 2 * lg_exchange_len(d) + 256 + (size_t)lg_points(d) / 2;
+}
+
+// Workgroups of a launch over n jobs that gets a share of the CUs: whole gangs
+// in equal numbers on the eight XCDs.
+static constexpr int LG_MAX_WG = 256;        // one workgroup per CU
+static inline int lg_workgroups(int n, double share) {
+    const int want = (LG_G * n + LG_MIN_WG - 1) / LG_MIN_WG * LG_MIN_WG;
+    int most = (int)(share * (LG_MAX_WG / LG_MIN_WG) + 0.5) * LG_MIN_WG;
+    if (most < LG_MIN_WG) most = LG_MIN_WG;
+    return want < most ? want : most;
+}
+static inline void lg_ctl_init(void* p, int njobs, int nwg) {
+    memset(p, 0, lg_ctl_bytes(njobs, nwg));
+    GangCtl* c = (GangCtl*)p;
+    c->njobs = (unsigned)njobs;
+    c->n_wg = (unsigned)nwg;
+}
+
+// Launches of a class over the instances d (job i is d[i]; device memory for a
+// solve, host memory for a single right-hand side or record, whose instance
+// travels with the launch), control block ctl (lg_ctl_init) and the gangs'
+// twiddle table tw.  False: no such kernel.
+struct GangLaunch {
+    int cls, nwg;
+    GangCtl* ctl;
+    const DInst* d;
+    const double2* tw;
+    hipStream_t s;
+};
+bool lg_field_solve(const GangLaunch& l, bool stream);
+bool lg_field_rhs(const GangLaunch& l, int* status);
+bool lg_field_stats(const GangLaunch& l, double z, double dz, int* status);
+bool lg_raman_solve(const GangLaunch& l, bool stream);  // field grids with a Raman response
+bool lg_raman_rhs(const GangLaunch& l, int* status);
+bool lg_env_solve(const GangLaunch& l, bool stream);
+bool lg_env_rhs(const GangLaunch& l, int* status);
+bool lg_env_stats(const GangLaunch& l, double z, double dz, int* status);
