@@ -216,8 +216,9 @@ int lh_solve_stream(lh_ctx *ctx, double *Ew_inout, const lh_rk_opts *opts, lh_ou
                     lh_stats *stats);
 
 /* Batched solve: n independent instances (each its own grid, constants, step
- * size control and status) in one persistent launch per grid class, one
- * workgroup per instance.  Radial contexts (whose one instance fills the GPU)
+ * size control and status) in one persistent launch per grid class, a gang of
+ * four workgroups per instance (z-dependent fills: one workgroup), the
+ * expensive instances first.  Radial contexts (whose one instance fills the GPU)
  * are solved one after another by a graph-replayed per-step launch sequence.
  * Replaces the per-point loop of Scans.runscan src/Scans.jl:275-430.
  * Ew_inout[i]: instance i's field; saves[i] may be NULL; stats[i] per instance.
@@ -434,9 +435,9 @@ int lh_wisdom_forget(void);
  * serving loops, harnesses that forbid hipMalloc).  The same device solve as
  * lh_solve on one mode-averaged context (field or envelope grid), with the
  * solver's working memory -- the instance record, the run counters, the save
- * grid, the second state buffer, the seven stage vectors and the envelope
- * Raman stash -- in one fixed buffer of LH_NOALLOC_SCRATCH_BYTES per GPU,
- * which the library holds until the process ends.  The call allocates nothing
+ * grid, the states and the stage vectors -- in one fixed buffer per GPU, which
+ * the library holds until the process ends (LH_NOALLOC_SCRATCH_BYTES bounds
+ * the problem, see below).  The call allocates nothing
  * (device or host): set the context up beforehand (lh_create, and
  * lh_set_step_stats / lh_set_gradient if used).
  *   Ew_dev    device pointer, complex [n_omega]: initial field in, final state out

@@ -13,10 +13,16 @@
 // turns one into the other.  The cumulative integrals of the plasma response
 // exchange one record per run (32 of them), the norms one record per member.
 //
-// Why four: a right-hand side has a fixed number of exchanges (4 with plasma),
-// about 1.5 us each through L2 whatever the gang's size, so the gain per added
-// CU falls; with four members the working set of two gangs fits a CU's LDS, so
-// that one gang computes while the other waits.
+// What bounds it: latency.  A right-hand side is a chain of some twenty phases
+// (LDS passes, exchanges, scans), each shorter than 2 us; the vector ALUs are
+// busy 30 % of the time.  An exchange costs 0.7 to 0.9 us through L2 and a
+// right-hand side with plasma has four, whatever the gang's size, so the gain
+// per added CU falls: four members are a compromise between one propagation
+// alone and a sweep that fills the chip.  Measured against one workgroup per
+// instance (one MI355X): a propagation at Nto = 8192 18.4 → 11.1 ms, envelope
+// Nt = 8192 with Raman 274 → 89 ms, Nt = 16384 57.4 → 12.1 ms, a single
+// right-hand side at Nto = 16384 56 → 38 us; a 64-point sweep 41.6 → 19.6 ms,
+// 256 points 47.1 → 45.2 ms.
 //
 // Gangs form by themselves: every workgroup of a launch takes a ticket of its
 // XCD (HW_REG_XCC_ID), and four consecutive tickets are a gang, so members are

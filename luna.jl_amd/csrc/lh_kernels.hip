@@ -1,14 +1,17 @@
-// lh_kernels.hip -- MI355X (gfx950) kernels and C ABI for the propagation hot path.
+// lh_kernels.hip -- C ABI of the propagation hot path on MI355X (gfx950): contexts,
+// batches, streaming, plans; and the kernels that are not in lh_gang.h.
 //
-// Design: one workgroup (512 threads, 8 wave64s) owns one instance.  A right-hand-side
-// evaluation keeps the whole oversampled time series in LDS:
+// Mode-averaged instances run on gangs of four workgroups (lh_gang.h), those
+// with a z-dependent fill on one workgroup (lh_zdep.hip), radial ones as a
+// launch sequence (lh_radial.hip).  A right-hand side keeps its time series in
+// LDS:
 //   stage prologue (ȳ = y + Δz Σ B k, ·exp(LΔ)) → c2r pre-pack → inverse
 //   Stockham FFT → Kerr + PPT spline + three cumtrapz block scans + towin →
 //   forward FFT → r2c post-step, crop, normalisation → stage epilogue
 //   (·exp(-LΔ)) written to HBM.
 // The adaptive Dormand–Prince loop (controller, window filter, dense-output
-// saves) runs inside the same workgroup, so a whole propagation is one launch
-// and a batch of independent instances is one launch of many workgroups.
+// saves) runs inside the same launch, so a whole propagation is one launch and
+// a batch of independent instances is one launch per grid size.
 //
 // Reference semantics (file:line in the reference tree):
 //   TransModeAvg              src/NonlinearRHS.jl:362-387
