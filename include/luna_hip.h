@@ -299,7 +299,7 @@ int lh_set_gradient(lh_ctx *ctx, const lh_gradient_desc *g);
 /* PPT ionisation-rate table (set-up of PlasmaCumtrapz): ionrate_fun_PPT
  * (src/Ionisation.jl:317-390, φ :403-429) at n field values on the GPU, as
  * makePPTcache tabulates it (src/Ionisation.jl:185-200) before makePPTaccel
- * fits its log-rate spline.  One thread per field value. */
+ * fits its log-rate spline.  A group of lanes per field value. */
 typedef struct lh_ppt_desc {
     double ionpot;            /* ionisation potential (J)                        */
     double lambda0;           /* wavelength (m)                                   */

@@ -23,10 +23,11 @@ FLAGS = [
 ]
 
 
-# The gang kernels hold one long loop around every phase of a step; hoisting the
-# FP64 constants of its exponentials and powers out of it costs registers that
-# then spill (22 to 59 VGPRs against none; 5 % of a propagation at Nto = 8192).
-GANG_FLAGS = ["-mllvm", "-disable-machine-licm"]
+# The gang kernels hold one long loop around every phase of a step, the PPT
+# kernel one around its series; hoisting the FP64 constants of their exponentials
+# and powers out of it costs registers that then spill (gangs: 22 to 59 VGPRs
+# against none, 5 % of a propagation at Nto = 8192; PPT: 28 to 40).
+LOOP_FLAGS = ["-mllvm", "-disable-machine-licm"]
 
 H5_SRC = os.path.join(HERE, "csrc", "lh_h5.c")
 H5_OUT = os.path.join(OUT_DIR, "libluna_h5.so")
@@ -57,7 +58,7 @@ def build(verbose=False):
     os.makedirs(OUT_DIR, exist_ok=True)
     tag = f".tmp{os.getpid()}"
     objs = [os.path.join(OUT_DIR, os.path.basename(s).replace(".hip", ".o") + tag) for s in SRCS]
-    procs = [subprocess.Popen([HIPCC] + FLAGS + (GANG_FLAGS if "lh_gang" in s else []) + ["-c", "-o", o, s], stdout=subprocess.PIPE,
+    procs = [subprocess.Popen([HIPCC] + FLAGS + (LOOP_FLAGS if ("lh_gang" in s or "lh_ppt" in s) else []) + ["-c", "-o", o, s], stdout=subprocess.PIPE,
                               stderr=subprocess.PIPE, text=True) for s, o in zip(SRCS, objs)]
     failed = []
     for p, s in zip(procs, SRCS):

@@ -221,8 +221,8 @@ def ionrate_ppt_vec(ionpot, lam0, Z, l, E, sum_tol=1e-6, dalpha=0.0, alpha_ion=0
 
 def ppt_device_table(ionpot, lam0, Z, l, E, sum_tol=1e-6, dalpha=0.0, alpha_ion=0.0, occupancy=2,
                      Cnl=None, timing=None):
-    """The same rates computed on the GPU (``lh_ppt_table``: one thread per
-    field value, each running the converge_series loop itself)."""
+    """The same rates computed on the GPU (``lh_ppt_table``: a group of
+    lanes per field value runs the converge_series loop)."""
     import ctypes as C
     from . import _capi
     E = np.ascontiguousarray(E, dtype=float)
