@@ -40,6 +40,7 @@
 #include "../../include/luna_hip.h"
 #include "lh_core.h"
 #include "lh_gang_launch.h"
+#include "lh_hostcopy.h"
 
 static const long long LH_MAX_STEPS = 500000;  // default cap on step attempts per instance
 
@@ -1418,7 +1419,7 @@ int lh_get_saves(lh_ctx* c, double* saves, double* zsaves) {
     HIPCK(hipSetDevice(c->device));
     int n = c->result_save_n;
     if (saves && n > 0)
-        HIPCK(hipMemcpy(saves, c->saves, sizeof(double2) * (size_t)c->n_state * n, hipMemcpyDeviceToHost));
+        HIPCK(copy_to_host(saves, c->saves, sizeof(double2) * (size_t)c->n_state * n, c->device, c->stream));
     if (zsaves && n > 0) HIPCK(hipMemcpy(zsaves, c->zgrid, sizeof(double) * n, hipMemcpyDeviceToHost));
     return LH_OK;
 }
@@ -1604,11 +1605,17 @@ int lh_batch_solve_opts(lh_ctx* const* ctxs, int n, double* const* Ew, const lh_
         if (st) return st;
     }
     int want = 0;
+    HostPages pages;
     for (int i = 0; i < n; i++)
-        if (saves && saves[i]) want = 1;
+        if (saves && saves[i]) {
+            want = 1;
+            pages.add(saves[i], sizeof(double2) * (size_t)ctxs[i]->n_state * (size_t)std::max(opts[i].save_n, 0));
+        }
     std::vector<const lh_rk_opts*> op((size_t)n);
     for (int i = 0; i < n; i++) op[i] = opts + i;
+    pages.start();
     int st = batch_resident(ctxs, n, op.data(), want, stats);
+    pages.wait();
     if (st) return st;
     for (int i = 0; i < n && !st; i++) {
         st = lh_get_state(ctxs[i], Ew[i]);
@@ -2083,9 +2090,15 @@ int lh_batch_solve(lh_ctx* const* ctxs, int n, double* const* Ew, const lh_rk_op
         if (st) return st;
     }
     int want = 0;
+    HostPages pages;
     for (int i = 0; i < n; i++)
-        if (saves && saves[i]) want = 1;
+        if (saves && saves[i]) {
+            want = 1;
+            pages.add(saves[i], sizeof(double2) * (size_t)ctxs[i]->n_state * (size_t)std::max(o->save_n, 0));
+        }
+    pages.start();
     int st = lh_batch_solve_resident(ctxs, n, o, want, stats);
+    pages.wait();
     if (st) return st;
     for (int i = 0; i < n && !st; i++) {
         st = lh_get_state(ctxs[i], Ew[i]);
