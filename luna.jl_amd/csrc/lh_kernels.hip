@@ -861,9 +861,7 @@ static int rad_solve(lh_ctx* c, const lh_rk_opts* o, bool want_saves, hipStream_
     RadCtl h;
     rad_ctl_init(&h, o);
     h.rhs_evals = 1;
-    HIPCK(hipStreamSynchronize(s));
-    HIPCK(hipMemcpy(c->rargs, &a, sizeof(a), hipMemcpyHostToDevice));
-    HIPCK(hipMemcpy(c->rctl, &h, sizeof(h), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, a, h, c->rargs);
     HIPCK(hipMemcpyAsync(c->Y, c->Yin, sizeof(double2) * (size_t)c->n_state, hipMemcpyDeviceToDevice, s));
     rad_rhs_dispatch(c->rplan, c->d.grid_kind == LH_GRID_ENV, n_to, n_r, c->rargs, tw, -1, s);  // PreconStepper init: k1 = fbar(y0)
     HIPCK(hipGetLastError());
@@ -1131,8 +1129,7 @@ int lh_rhs_device(lh_ctx* c, void* nl_dev, const void* Ew_dev, double z, void* s
         a.rhs_out = (double2*)nl_dev;
         RadCtl h;
         rad_ctl_init(&h, nullptr);
-        HIPCK(hipMemcpyAsync(c->rargs + 1, &a, sizeof(a), hipMemcpyHostToDevice, s));
-        HIPCK(hipMemcpyAsync(c->rctl + 1, &h, sizeof(h), hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, a, h, c->rargs + 1);
         rad_rhs_dispatch(c->rplan, c->d.grid_kind == LH_GRID_ENV, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s);
     } else {
         DInst in = base_inst(c);
