@@ -9,7 +9,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", n) for n in ("lh_kernels.hip", "lh_gang_field.hip", "lh_gang_raman.hip",
-                                                "lh_gang_env.hip", "lh_fno.hip", "lh_ppt.hip")]
+                                                "lh_gang_env.hip", "lh_gang_dense.hip", "lh_fno.hip", "lh_ppt.hip")]
 OUT_DIR = os.path.join(HERE, "_build")
 OUT = os.path.join(OUT_DIR, "libluna_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

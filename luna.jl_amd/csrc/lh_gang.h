@@ -737,7 +737,7 @@ struct GSizes {
     static constexpr int N = (KIND == 0) ? M / 2 + 1 : M;     // state bins
     static constexpr int NPT = (NMAX + LH_T - 1) / LH_T;      // bins per thread
     static constexpr int CB = NPT <= 3 ? NPT : (KIND == 0) ? 3 : 2;  // of them in one round of loads
-    static constexpr int NC = (NPT + CB - 1) / CB;
+    static constexpr int CBD = (KIND == 0 && NPT >= 2) ? 2 : 1;      // in a dense kernel (half the registers)
     __device__ static __forceinline__ int count(int h) { return (KIND == 0 && h == 0) ? NB + 1 : NB; }
     // local bin p → (slot, q); k = res + 8q.  Field grids: p < S/2 is slot 0,
     // p < S slot 1, p = S (member 0) bin M/2.
@@ -1174,10 +1174,10 @@ __device__ __forceinline__ double2 g_rhs_bin(const SM& sm, const Gang& g, int p)
 // Persistent adaptive solve of one instance by a gang (Luna.run →
 // RK45.solve_precon).  Every member runs the same step control on the same
 // numbers.
-template <int KIND, int M, bool STREAM, bool RAMAN, class SM>
+template <int KIND, int M, bool STREAM, bool RAMAN, bool DENSE, class SM>
 __device__ __forceinline__ void g_solve(const DInst& in, SM& sm, Gang& g) {
     using Z = GSizes<KIND, M>;
-    constexpr int N = Z::N, CB = Z::CB, NC = Z::NC;
+    constexpr int N = Z::N, CB = DENSE ? Z::CBD : Z::CB, NC = (Z::NPT + CB - 1) / CB;
     const int h = g.h, nb = Z::count(h);
     KSet K{gl(in.K) + (size_t)h * Z::GSTR, in.kstride, 0, 6};
     double2* const Fv = K[LG_F];
@@ -1630,9 +1630,13 @@ __device__ __forceinline__ void gang_area(Gang& g, const DInst& in) {
     g.P = g.rec + 512;
 }
 
-template <int KIND, int M, bool STREAM, bool RAMAN>
-__global__ __launch_bounds__(LH_T) void lh_gang_solve(GangCtl* ctl, const DInst* insts,
-                                                           const double2* __restrict__ twg) {
+// DENSE: compiled for two workgroups per CU (128 registers; 115 of the field
+// kernel's values at Nto = 16384 spill, most of them around the transform
+// passes; 204 with three bins per thread in a round of loads).  The same source,
+// so the same bits; the loads of a round alone are grouped differently.
+template <int KIND, int M, bool STREAM, bool RAMAN, bool DENSE = false>
+__global__ __launch_bounds__(LH_T, DENSE ? 4 : 1) void lh_gang_solve(GangCtl* ctl, const DInst* insts,
+                                                                     const double2* __restrict__ twg) {
     using SM = typename GLds<KIND, M, RAMAN>::T;
     __shared__ SM sm;
     gtw_load(sm.tw, twg);
@@ -1640,7 +1644,7 @@ __global__ __launch_bounds__(LH_T) void lh_gang_solve(GangCtl* ctl, const DInst*
     gang_loop<false>(ctl, sm, g, [&](int job) {
         const DInst& in = insts[job];
         gang_area(g, in);
-        g_solve<KIND, M, STREAM, RAMAN>(in, sm, g);
+        g_solve<KIND, M, STREAM, RAMAN, DENSE>(in, sm, g);
     });
 }
 
@@ -1734,6 +1738,12 @@ static bool lg_launch_solve(const GangLaunch& l, bool stream) {
         hipLaunchKernelGGL((lh_gang_solve<KIND, M, true, RAMAN>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
     else
         hipLaunchKernelGGL((lh_gang_solve<KIND, M, false, RAMAN>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
+    return true;
+}
+template <int KIND, int M>
+static bool lg_launch_dense(const GangLaunch& l) {
+    static_assert(2 * sizeof(typename GLds<KIND, M, false>::T) <= 160 * 1024, "two workgroups per CU");
+    hipLaunchKernelGGL((lh_gang_solve<KIND, M, false, false, true>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
     return true;
 }
 template <int KIND, int M, bool RAMAN>

@@ -44,16 +44,22 @@ static inline size_t lg_area_len(const lh_desc& d) {  // complex points of the e
 }
 
 // Workgroups of a launch over n jobs that gets a share of the CUs: whole gangs
-// in equal numbers on the eight XCDs, one workgroup per CU (the registers of
-// two would have to fit 128 per lane: 80 to 200 of them then spill, and a
-// propagation alone took 10 % more time for 15 % more throughput).
+// in equal numbers on the eight XCDs, one workgroup per CU, two of a dense kernel.
 static constexpr int LG_MAX_WG = 256;        // one workgroup per CU
-static inline int lg_workgroups(int n, double share) {
+static inline int lg_workgroups(int n, double share, bool dense) {
     const int want = (LG_G * n + LG_MIN_WG - 1) / LG_MIN_WG * LG_MIN_WG;
-    int most = (int)(share * (LG_MAX_WG / LG_MIN_WG) + 0.5) * LG_MIN_WG;
+    int most = (int)(share * ((dense ? 2 : 1) * LG_MAX_WG / LG_MIN_WG) + 0.5) * LG_MIN_WG;
     if (most < LG_MIN_WG) most = LG_MIN_WG;
     return want < most ? want : most;
 }
+// Instances in a batch above which it runs on dense kernels, where a class has
+// one.  A gang on half the registers and half a CU per member takes 1.6 times as
+// long for a step, two of them do 1.25 times as much: better once there are two
+// to three instances for each of the 64 gangs, before that the longest instance
+// decides.  ms for n propagations of 0.4 m (half Nto = 8192, half 16384), one
+// workgroup per CU / two: 128 23.2/29.0, 160 27.7/29.7, 192 34.4/30.3, 224
+// 38.8/33.2, 256 44.6/40.0; 384 of 0.2 m 35.3/34.0.
+static constexpr int LG_DENSE_ABOVE = 176;
 static inline void lg_ctl_init(void* p, int njobs, int nwg) {
     memset(p, 0, lg_ctl_bytes(njobs, nwg));
     GangCtl* c = (GangCtl*)p;
@@ -73,6 +79,8 @@ struct GangLaunch {
     hipStream_t s;
 };
 bool lg_field_solve(const GangLaunch& l, bool stream);
+bool lg_has_dense(int cls, bool raman);
+bool lg_dense_solve(const GangLaunch& l);
 bool lg_field_rhs(const GangLaunch& l, int* status);
 bool lg_field_stats(const GangLaunch& l, double z, double dz, int* status);
 bool lg_raman_solve(const GangLaunch& l, bool stream);  // field grids with a Raman response

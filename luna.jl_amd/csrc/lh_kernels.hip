@@ -1486,7 +1486,8 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     }
     std::stable_sort(by_cost.begin(), by_cost.end(), [&](int a, int b) { return cost[a] > cost[b]; });
     double group_cost[NG] = {0}, all_cost = 0.0;
-    int nwg[NG] = {0}, last_gang = -1;
+    int nwg[NG] = {0}, last_gang = -1, n_gang = 0;
+    bool dense[NG] = {false};
     {
         int fill[NG] = {0};
         for (int i : by_cost) {
@@ -1495,14 +1496,18 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
             if (c < V_ZDEP * LH_NCLASS && c != LH_CLASS_RADIAL) group_cost[c] += cost[i], all_cost += cost[i];
         }
     }
+    for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
+        if (c != LH_CLASS_RADIAL) n_gang += count[c];
+    for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
+        dense[c] = n_gang > LG_DENSE_ABOVE && lg_has_dense(c % LH_NCLASS, c >= V_RAMAN * LH_NCLASS);
     for (int gi = 0; gi < NG; gi++) {
         const int c = (gi % N_VAR) * LH_NCLASS + order[gi / N_VAR];
         if (!count[c] || c >= V_ZDEP * LH_NCLASS || c == LH_CLASS_RADIAL) continue;
         const double share = all_cost > 0.0 ? group_cost[c] / all_cost : 1.0;
-        nwg[c] = lg_workgroups(count[c], share);
+        nwg[c] = lg_workgroups(count[c], share, dense[c]);
         last_gang = c;
     }
-    if (last_gang >= 0) nwg[last_gang] = lg_workgroups(count[last_gang], 1.0);
+    if (last_gang >= 0) nwg[last_gang] = lg_workgroups(count[last_gang], 1.0, dense[last_gang]);
     // one device block: the instances' records, each class's control block, the
     // run counters
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -1547,9 +1552,8 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         } else if (var == V_ZDEP) {
             launch_zdep(cls, count[c], dinst + first[c], tw16, cs);
         } else {
-            if (!launch_solve({cls, nwg[c], (GangCtl*)(dblk + ctl_off[c]), dinst + first[c], tw, cs},
-                              var == V_RAMAN, false))
-                st = LH_E_ARG;
+            const GangLaunch l{cls, nwg[c], (GangCtl*)(dblk + ctl_off[c]), dinst + first[c], tw, cs};
+            if (!(dense[c] ? lg_dense_solve(l) : launch_solve(l, var == V_RAMAN, false))) st = LH_E_ARG;
         }
         if (st || hipGetLastError() != hipSuccess || hipEventRecord(t1[c], cs) != hipSuccess ||
             hipEventRecord(done[c], cs) != hipSuccess || hipStreamWaitEvent(s0, done[c], 0) != hipSuccess)
