@@ -41,6 +41,7 @@
 #include "lh_core.h"
 #include "lh_gang_launch.h"
 #include "lh_hostcopy.h"
+#include "lh_zdep.h"
 
 static const long long LH_MAX_STEPS = 500000;  // default cap on step attempts per instance
 
@@ -182,9 +183,6 @@ static bool launch_stats(const GangLaunch& l, double z, double dz, int* status) 
 
 // Radially symmetric transform: per-column kernels and FP64 MFMA contraction.
 #include "lh_radial.hip"
-
-// Propagation with a z-dependent fill.
-#include "lh_zdep.hip"
 
 // ==========================================================================
 // Host side: contexts, constant upload, launches (C ABI, include/luna_hip.h)

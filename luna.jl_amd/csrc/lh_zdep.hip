@@ -1,8 +1,8 @@
 // lh_zdep.hip -- propagation with a z-dependent fill (pressure gradient, taper),
 // one workgroup per instance (gfx950).
 //
-// Included by lh_kernels.hip.  The constant-fill instances run on gangs of
-// workgroups (lh_gang.hip); these stay on one workgroup and on its order of
+// The constant-fill instances run on gangs of
+// workgroups (lh_gang.h); these stay on one workgroup and on its order of
 // operations, because their operator amplifies rounding: β1(z) is a 9-point
 // difference of β ≈ 8e6 rad/m over a step h, so one unit in the last place of
 // a single β moves the phase of the field by 1e-9 to 1e-8 over a propagation.
@@ -10,6 +10,8 @@
 // positions z by a relative 1e-13 through the error estimate, which is enough
 // to flip such a unit at some z: the same solver on gangs took 19.4 ms instead
 // of 42.6 for a 0.5 m propagation at Nto = 16384, but landed 5e-8 away.
+#include "lh_core.h"
+#include "lh_zdep.h"
 
 // Epilogues of a transform: called with v[i] = the RHS of bin
 // k = (the thread's index) + i·LH_T.
@@ -90,35 +92,39 @@ __device__ __forceinline__ void stage_prologue(const DInst& in, Smem& sm, const 
 }
 
 // Re-evaluate the z-dependent constants at z (make_prop!(linop!) evaluates
-// linop!(out, t2) whenever t2 changes): ρ(z) and β1(z) on thread 0, then per
+// linop!(out, t2) whenever t2 changes): ρ(z) and β1(z) on the first wavefront,
+// one stencil point per lane and the sum in the points' order, then per
 // bin the operator -i(ω/c·conj_clamp(neff) - ω β1) (src/LinearOps.jl:337-358,
 // 254) and the output factor sc_f·pre/β·√Aeff·ωwin (β = ω/c·Re neff),
 // written to gl(in.zL) / gl(in.zOF).  Returns ρ(z) and the Kerr factor ρ ε0 γ3.
 template <class Smem>
 __device__ __forceinline__ void zg_refresh(const DInst& in, Smem& sm, double z, double& rho, double& kfac) {
     const int tid = fresh_tid();
-    if (tid == 0) {
+    if (tid < 64) {
         const double p = zg_pressure(in, z);
         const double r = cspline_uniform(gl(in.zd), in.zd_n, gl(in.zd)[0].x, gl(in.zd)[in.zd_n - 1].x, p);
         // β1 = Modes.dispersion(mode, 1, ω0, z): β(ω) = ω/c·Re neff(mode, ω; z)
         // with neff's own clamp (src/Capillary.jl:162-186)
         const double a = in.ztaper ? zg_radius(in, z) : 0.0;
-        double acc = 0.0;
-        for (int j = 0; j < 9; j++) {
-            const double* f = gl(in.zfd) + 4 * j;
-            const double sc = sqrt(1 + f[1] * r);
-            double2 nwj = make_double2(f[2], f[3]);
-            if (in.ztaper) {
-                const double* t = gl(in.zfdt) + 3 * j;
-                nwj = zg_nwg_taper(in, t[0], make_double2(t[1], t[2]), a);
-            }
-            double nr = zg_neff(in, sc * sc, nwj).x;
-            if (in.zg_model == 0 && nr < 1e-3) nr = 1e-3;
-            acc += c_fd8[j] * (f[0] / LH_CLIGHT * nr);
+        const int j = min(tid, 8);
+        const double* f = gl(in.zfd) + 4 * j;
+        const double sc = sqrt(1 + f[1] * r);
+        double2 nwj = make_double2(f[2], f[3]);
+        if (in.ztaper) {
+            const double* t = gl(in.zfdt) + 3 * j;
+            nwj = zg_nwg_taper(in, t[0], make_double2(t[1], t[2]), a);
         }
-        sm.zs[0] = r;
-        sm.zs[1] = acc / in.zfd_h;
-        sm.zs[2] = a;
+        double nr = zg_neff(in, sc * sc, nwj).x;
+        if (in.zg_model == 0 && nr < 1e-3) nr = 1e-3;
+        const double beta = f[0] / LH_CLIGHT * nr;
+        double acc = 0.0;
+#pragma unroll
+        for (int i = 0; i < 9; i++) acc = fma(c_fd8[i], lane_value(beta, i), acc);
+        if (tid == 0) {
+            sm.zs[0] = r;
+            sm.zs[1] = acc / in.zfd_h;
+            sm.zs[2] = a;
+        }
     }
     __syncthreads();
     rho = sm.zs[0];
@@ -126,26 +132,50 @@ __device__ __forceinline__ void zg_refresh(const DInst& in, Smem& sm, double z, 
     const double a = sm.zs[2];
     const double sqrt_aeff = in.ztaper ? a * in.zsqrt_intg : in.zsqrt_aeff;  // Aeff(z) = a(z)²·aeff_intg
     kfac = rho * LH_EPS0 * in.kerr_gamma3;
-    for (int k = tid; k < in.n_omega; k += LH_T) {
-        double2 L = make_double2(0.0, 0.0), of = make_double2(in.sc_f, 0.0);
-        if (gl(in.zsidx)[k]) {
-            const double w = gl(in.st_omega)[k];
-            const double sc = sqrt(1 + gl(in.zgam)[k] * rho);  // coren(ω; z)^2
-            const double2 nw = in.ztaper ? zg_nwg_taper(in, gl(in.zU)[k], gl(in.zV)[k], a) : static_cast<const double2*>(gl(in.znwg))[k];
-            const double2 n = zg_neff(in, sc * sc, nw);
-            const double ncr = (n.x < 1e-3) ? 1e-3 : n.x;  // conj_clamp
-            const double lim = 3000 * LH_CLIGHT / w;
-            const double nci = -((n.y < 0.0) ? 0.0 : (n.y > lim ? lim : n.y));
-            const double wc = w / LH_CLIGHT;
-            const double zr = wc * ncr - w * b1, zi = wc * nci;
-            L = make_double2(zi, -zr);
-            const double beta = wc * n.x;
-            const double2 pre = gl(in.zpre)[k];
-            const double nfx = pre.x / beta * sqrt_aeff, nfy = pre.y / beta * sqrt_aeff;
-            of = make_double2((in.sc_f * nfx) * gl(in.omega_win)[k], (in.sc_f * nfy) * gl(in.omega_win)[k]);
+    // three bins per round: their loads are in flight together (a bin at a time
+    // waited for zsidx, then for the rest, nine times per refresh at Nto = 16384:
+    // 40.9 → 38.2 ms for a 0.5 m propagation; one stencil point per lane above
+    // instead of nine in a row: 42.9 → 40.9 ms; the same bits)
+    constexpr int CB = 3;
+    const int N = in.n_omega;
+#pragma unroll 1
+    for (int k0 = tid; k0 < N; k0 += CB * LH_T) {
+        double w[CB], gam[CB], win[CB], U[CB];
+        double2 nw[CB], pre[CB];
+        bool live[CB];
+#pragma unroll
+        for (int i = 0; i < CB; i++) {
+            const int k = min(k0 + i * LH_T, N - 1);
+            live[i] = gl(in.zsidx)[k];
+            w[i] = gl(in.st_omega)[k];
+            gam[i] = gl(in.zgam)[k];
+            win[i] = gl(in.omega_win)[k];
+            pre[i] = static_cast<const double2*>(gl(in.zpre))[k];
+            U[i] = in.ztaper ? gl(in.zU)[k] : 0.0;
+            nw[i] = in.ztaper ? static_cast<const double2*>(gl(in.zV))[k] : static_cast<const double2*>(gl(in.znwg))[k];
         }
-        gl(in.zL)[k] = L;
-        gl(in.zOF)[k] = of;
+#pragma unroll
+        for (int i = 0; i < CB; i++) {
+            const int k = k0 + i * LH_T;
+            if (k >= N) break;
+            double2 L = make_double2(0.0, 0.0), of = make_double2(in.sc_f, 0.0);
+            if (live[i]) {
+                const double sc = sqrt(1 + gam[i] * rho);  // coren(ω; z)^2
+                const double2 nwk = in.ztaper ? zg_nwg_taper(in, U[i], nw[i], a) : nw[i];
+                const double2 n = zg_neff(in, sc * sc, nwk);
+                const double ncr = (n.x < 1e-3) ? 1e-3 : n.x;  // conj_clamp
+                const double lim = 3000 * LH_CLIGHT / w[i];
+                const double nci = -((n.y < 0.0) ? 0.0 : (n.y > lim ? lim : n.y));
+                const double wc = w[i] / LH_CLIGHT;
+                const double zr = wc * ncr - w[i] * b1, zi = wc * nci;
+                L = make_double2(zi, -zr);
+                const double beta = wc * n.x;
+                const double nfx = pre[i].x / beta * sqrt_aeff, nfy = pre[i].y / beta * sqrt_aeff;
+                of = make_double2((in.sc_f * nfx) * win[i], (in.sc_f * nfy) * win[i]);
+            }
+            gl(in.zL)[k] = L;
+            gl(in.zOF)[k] = of;
+        }
     }
     __syncthreads();
 }
@@ -649,7 +679,7 @@ __global__ __launch_bounds__(LH_T) void lh_zdep_solve(const DInst* insts, const 
     zdep_solve<MO, MC, SmemT<MO>>(insts[blockIdx.x], sm);
 }
 
-static void launch_zdep(int cls, int n, const DInst* dinst, const double2* tw, hipStream_t s) {
+void launch_zdep(int cls, int n, const DInst* dinst, const double2* tw, hipStream_t s) {
     switch (cls) {
         case LH_CLASS_16384: hipLaunchKernelGGL((lh_zdep_solve<8192, 4096>), dim3(n), dim3(LH_T), 0, s, dinst, tw); break;
         case LH_CLASS_8192: hipLaunchKernelGGL((lh_zdep_solve<4096, 2048>), dim3(n), dim3(LH_T), 0, s, dinst, tw); break;
