@@ -736,7 +736,9 @@ struct GSizes {
     static constexpr int MC = (KIND == 0) ? M / 2 : M;        // filter transform
     static constexpr int N = (KIND == 0) ? M / 2 + 1 : M;     // state bins
     static constexpr int NPT = (NMAX + LH_T - 1) / LH_T;      // bins per thread
-    static constexpr int CB = NPT <= 3 ? NPT : (KIND == 0) ? 3 : 2;  // of them in one round of loads
+    // of them in one round of loads (as many as the registers hold: envelope grids
+    // of 16384 points with four instead of two 12.15 → 11.84 ms for 0.15 m)
+    static constexpr int CB = NPT <= 4 ? NPT : (KIND == 0) ? 3 : 4;
     static constexpr int CBD = (KIND == 0 && NPT >= 2) ? 2 : 1;      // in a dense kernel (half the registers)
     __device__ static __forceinline__ int count(int h) { return (KIND == 0 && h == 0) ? NB + 1 : NB; }
     // local bin p → (slot, q); k = res + 8q.  Field grids: p < S/2 is slot 0,
