@@ -739,7 +739,7 @@ struct GSizes {
     // of them in one round of loads (as many as the registers hold: envelope grids
     // of 16384 points with four instead of two 12.15 → 11.84 ms for 0.15 m)
     static constexpr int CB = NPT <= 4 ? NPT : (KIND == 0) ? 3 : 4;
-    static constexpr int CBD = (KIND == 0 && NPT >= 2) ? 2 : 1;      // in a dense kernel (half the registers)
+    static constexpr int CBD = NPT >= 2 ? 2 : 1;              // in a dense kernel (half the registers)
     __device__ static __forceinline__ int count(int h) { return (KIND == 0 && h == 0) ? NB + 1 : NB; }
     // local bin p → (slot, q); k = res + 8q.  Field grids: p < S/2 is slot 0,
     // p < S slot 1, p = S (member 0) bin M/2.
@@ -1742,10 +1742,10 @@ static bool lg_launch_solve(const GangLaunch& l, bool stream) {
         hipLaunchKernelGGL((lh_gang_solve<KIND, M, false, RAMAN>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
     return true;
 }
-template <int KIND, int M>
+template <int M>
 static bool lg_launch_dense(const GangLaunch& l) {
-    static_assert(2 * sizeof(typename GLds<KIND, M, false>::T) <= 160 * 1024, "two workgroups per CU");
-    hipLaunchKernelGGL((lh_gang_solve<KIND, M, false, false, true>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
+    static_assert(2 * sizeof(typename GLds<0, M, false>::T) <= 160 * 1024, "two workgroups per CU");
+    hipLaunchKernelGGL((lh_gang_solve<0, M, false, false, true>), dim3(l.nwg), dim3(LH_T), 0, l.s, l.ctl, l.d, l.tw);
     return true;
 }
 template <int KIND, int M, bool RAMAN>

@@ -2,7 +2,7 @@
 // batches, streaming, plans; and the kernels that are not in lh_gang.h.
 //
 // Mode-averaged instances run on gangs of four workgroups (lh_gang.h), those
-// with a z-dependent fill on one workgroup (lh_zdep.hip), radial ones as a
+// with a z-dependent fill on one workgroup (lh_solo.hip), radial ones as a
 // launch sequence (lh_radial.hip).  A right-hand side keeps its time series in
 // LDS:
 //   stage prologue (ȳ = y + Δz Σ B k, ·exp(LΔ)) → c2r pre-pack → inverse
@@ -41,7 +41,7 @@
 #include "lh_core.h"
 #include "lh_gang_launch.h"
 #include "lh_hostcopy.h"
-#include "lh_zdep.h"
+#include "lh_solo.h"
 
 static const long long LH_MAX_STEPS = 500000;  // default cap on step attempts per instance
 
@@ -561,7 +561,7 @@ static DInst base_inst(const lh_ctx* c) {
         in.zfdt = c->zfdt;
         in.zL = c->zL;
         in.zOF = c->zOF;
-        in.linop = c->zL;  // refreshed in place at every new z (lh_zdep.hip)
+        in.linop = c->zL;  // refreshed in place at every new z (lh_solo.hip)
         in.outfac = c->zOF;
     }
     return in;
@@ -586,7 +586,14 @@ static GangLaunch launch1_of(const lh_ctx* c, unsigned char* at, const double2* 
 // its control block and exchange area, so one on another stream than the last
 // waits for that one.
 static int rhs_launch_of(lh_ctx* c, const DInst* in, const double2* tw, hipStream_t s, GangLaunch* l) {
-    if (c->rhs_stream && c->rhs_stream != s) {
+    // a stream under capture neither waits for work outside its graph nor is
+    // waited for: the caller orders a graph's replays with its other calls
+    const auto capturing = [](hipStream_t q) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(q, &cs) != hipSuccess) (void)hipGetLastError();
+        return cs != hipStreamCaptureStatusNone;
+    };
+    if (c->rhs_stream && c->rhs_stream != s && !capturing(s) && !capturing(c->rhs_stream)) {
         if (!c->rhs_ev) HIPCK(hipEventCreateWithFlags(&c->rhs_ev, hipEventDisableTiming));
         if (hipEventRecord(c->rhs_ev, c->rhs_stream) != hipSuccess || hipStreamWaitEvent(s, c->rhs_ev, 0) != hipSuccess) {
             (void)hipGetLastError();  // the caller has destroyed that stream
@@ -687,6 +694,46 @@ static double class_us(int cls) {
 static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
     const double x = fabs(c->amp * c->d.density * c->d.gamma3) * (o->zmax - o->z0);
     return isfinite(x) ? x * class_us(ctx_class(c)) : 0.0;
+}
+
+// Whether the constant-fill field instances of a batch run on one workgroup each
+// (lh_solo.hip) instead of on gangs.  Both ways are priced with the estimated
+// lengths of their runs: alone, the slowest instance or the work over the CUs
+// decides; on gangs the work does.  µs per right-hand side: one workgroup 23.4,
+// 37.4, 63.7 at Nto = 4096, 8192, 16384; gangs, per instance on the whole chip,
+// 0.275, 0.31, 0.455 at one workgroup per CU and 0.241, 0.26, 0.382 on dense
+// kernels.  256 equal instances: 3.8, 6.1, 10.4 ms alone against 10.1, 10.9, 16.0
+// on gangs; a sweep of 256 whose lengths spread by a factor of ten (mean half the
+// longest): 51 against 40.  The rule depends on the batch alone, so a batch gives
+// the same bits every time; the two ways agree to rounding.
+static bool solo_class(const lh_ctx* c) {
+    const int cls = ctx_class(c);
+    return c->d.transform == LH_TRANS_MODEAVG && !c->zg_on && !c->d.raman &&
+           (cls == LH_CLASS_16384 || cls == LH_CLASS_8192 || cls == LH_CLASS_4096);
+}
+static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
+    const bool dense = n > LG_DENSE_ABOVE;
+    double longest = 0.0, alone = 0.0, gangs = 0.0;
+    int m = 0, zero = 0;
+    for (int pass = 0; pass < 2; pass++) {
+        for (int i = 0; i < n; i++) {
+            if (!solo_class(ctxs[i])) continue;
+            const int cls = ctx_class(ctxs[i]);
+            double w = solve_cost(ctxs[i], op[i]) / class_us(cls);
+            if (pass == 0) {
+                m++;
+                zero += (w == 0.0);
+                continue;
+            }
+            if (zero == m) w = 1.0;  // linear runs: equal lengths
+            const double us = cls == LH_CLASS_16384 ? 63.7 : cls == LH_CLASS_8192 ? 37.4 : 23.4;
+            longest = std::max(longest, w * us);
+            alone += w * us / LG_MAX_WG;
+            gangs += w * (dense ? (cls == LH_CLASS_16384 ? 0.382 : cls == LH_CLASS_8192 ? 0.26 : 0.241)
+                                : (cls == LH_CLASS_16384 ? 0.455 : cls == LH_CLASS_8192 ? 0.31 : 0.275));
+        }
+    }
+    return m > 0 && std::max(longest, alone) < gangs;
 }
 
 static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, DInst* in, lh_stats* dstats_slot,
@@ -1422,7 +1469,7 @@ int lh_get_saves(lh_ctx* c, double* saves, double* zsaves) {
 // One stream per (device, size class and kernel) for the batched launches, created on
 // first use and kept for the process (default priority).
 static std::mutex g_cls_mu;
-static hipStream_t g_cls_stream[64][3 * LH_NCLASS];
+static hipStream_t g_cls_stream[64][4 * LH_NCLASS];
 
 static int class_stream(int dev, int c, hipStream_t* out) {
     if (dev < 0 || dev >= 64) return LH_E_ARG;
@@ -1453,18 +1500,20 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     if (!st) st = twiddles(dev, &tw16);
     if (st) return st;
     // group instances by size class and kernel (gangs, gangs with a field-grid
-    // Raman response, one workgroup for z-dependent fills); each group is one
+    // Raman response, one workgroup for z-dependent fills and for even batches);
+    // each group is one
     // persistent launch on its own stream so the groups run concurrently.  The
     // larger grids come first: their gangs take the CUs, the others' workgroups
     // follow as those run out of jobs.  Radial contexts block the host and come
     // last.
-    enum { V_GANG, V_RAMAN, V_ZDEP, N_VAR };
+    const bool solo = solo_pays(ctxs, op, n);
+    enum { V_GANG, V_RAMAN, V_ZDEP, V_SOLO, N_VAR };
     constexpr int NG = N_VAR * LH_NCLASS;
     static const int order[LH_NCLASS] = {LH_CLASS_32768, LH_CLASS_ENV16384, LH_CLASS_16384, LH_CLASS_ENV8192,
                                          LH_CLASS_8192,  LH_CLASS_ENV4096,  LH_CLASS_4096,  LH_CLASS_RADIAL};
     auto group_of = [&](const lh_ctx* c) {
         const bool fr = c->d.transform == LH_TRANS_MODEAVG && c->d.grid_kind == LH_GRID_REAL && c->d.raman;
-        return (c->zg_on ? V_ZDEP : fr ? V_RAMAN : V_GANG) * LH_NCLASS + ctx_class(c);
+        return (c->zg_on ? V_ZDEP : fr ? V_RAMAN : (solo && solo_class(c)) ? V_SOLO : V_GANG) * LH_NCLASS + ctx_class(c);
     };
     int count[NG] = {0}, first[NG] = {0};
     for (int i = 0; i < n; i++) count[group_of(ctxs[i])]++;
@@ -1547,8 +1596,8 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
                 if (ctx_class(ctxs[i]) == LH_CLASS_RADIAL)
                     st = rad_solve(ctxs[i], op[i], want_saves != 0, cs, &rad_stats[i]);
             if (st) break;
-        } else if (var == V_ZDEP) {
-            launch_zdep(cls, count[c], dinst + first[c], tw16, cs);
+        } else if (var == V_ZDEP || var == V_SOLO) {
+            launch_solo(cls, count[c], dinst + first[c], tw16, cs, var == V_ZDEP);
         } else {
             const GangLaunch l{cls, nwg[c], (GangCtl*)(dblk + ctl_off[c]), dinst + first[c], tw, cs};
             if (!(dense[c] ? lg_dense_solve(l) : launch_solve(l, var == V_RAMAN, false))) st = LH_E_ARG;
@@ -2063,7 +2112,7 @@ int lh_solve_noalloc(lh_ctx* c, void* Ew_dev, const lh_rk_opts* o, void* saves_d
     }
     const GangLaunch l = launch1_of(c, base + L.inst, tw, s);
     if (c->zg_on)
-        launch_zdep(cls, 1, l.d, tw16, s);
+        launch_solo(cls, 1, l.d, tw16, s, true);
     else if (!launch_solve(l, c->d.raman != 0, false))
         return LH_E_ARG;
     HIPCK(hipGetLastError());

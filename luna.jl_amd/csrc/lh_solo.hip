@@ -1,17 +1,22 @@
-// lh_zdep.hip -- propagation with a z-dependent fill (pressure gradient, taper),
-// one workgroup per instance (gfx950).
+// lh_solo.hip -- propagation on a field grid, one workgroup per instance (gfx950).
 //
-// The constant-fill instances run on gangs of
-// workgroups (lh_gang.h); these stay on one workgroup and on its order of
-// operations, because their operator amplifies rounding: β1(z) is a 9-point
-// difference of β ≈ 8e6 rad/m over a step h, so one unit in the last place of
-// a single β moves the phase of the field by 1e-9 to 1e-8 over a propagation.
-// Any other order of operations in the right-hand side shifts the step
-// positions z by a relative 1e-13 through the error estimate, which is enough
-// to flip such a unit at some z: the same solver on gangs took 19.4 ms instead
-// of 42.6 for a 0.5 m propagation at Nto = 16384, but landed 5e-8 away.
+// Two kinds of instances run here instead of on gangs of workgroups (lh_gang.h).
+//
+// z-dependent fills (pressure gradient, taper) stay on this order of operations,
+// because their operator amplifies rounding: β1(z) is a 9-point difference of
+// β ≈ 8e6 rad/m over a step h, so one unit in the last place of a single β moves
+// the phase of the field by 1e-9 to 1e-8 over a propagation.  Any other order of
+// operations in the right-hand side shifts the step positions z by a relative
+// 1e-13 through the error estimate, which is enough to flip such a unit at some
+// z: the same solver on gangs took 19.4 ms instead of 42.6 for a 0.5 m
+// propagation at Nto = 16384, but landed 5e-8 away.
+//
+// Large even batches: a gang exchanges its series through the L2 and waits at
+// barriers, a workgroup alone does neither, so with an instance for every CU and
+// about equal lengths one workgroup each does 1.5 to 2.6 times as much per
+// second (solo_pays in lh_kernels.hip has the rule).
 #include "lh_core.h"
-#include "lh_zdep.h"
+#include "lh_solo.h"
 
 // Epilogues of a transform: called with v[i] = the RHS of bin
 // k = (the thread's index) + i·LH_T.
@@ -366,8 +371,8 @@ __device__ __forceinline__ void stats_time(const DInst& in, Smem& sm, double s0,
 }
 
 // Adaptive solve of one instance (Luna.run → RK45.solve_precon).
-template <int MO, int MC, class Smem>
-__device__ __forceinline__ void zdep_solve(const DInst& in, Smem& sm) {
+template <int MO, int MC, bool ZDEP, class Smem>
+__device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
     constexpr int N = Bins<MO>::N, NPT = Bins<MO>::NPT;
     KSet K{gl(in.K), in.kstride, 0, 6};
     double2* const Y0 = gl(in.Y);
@@ -383,7 +388,7 @@ __device__ __forceinline__ void zdep_solve(const DInst& in, Smem& sm) {
     // density and Kerr factor of the current z, re-evaluated with the operator at
     // every new z
     double rho = in.density, kfac = in.kerr_fac;
-    zg_refresh(in, sm, in.z0, rho, kfac);
+    if constexpr (ZDEP) zg_refresh(in, sm, in.z0, rho, kfac);
 
     // PreconStepper init: k1 = fbar(y0, t, t)
     stage_prologue<MO, Smem>(in, sm, Y, K, 0, 0.0, 0.0, 0.0);
@@ -403,18 +408,20 @@ __device__ __forceinline__ void zdep_solve(const DInst& in, Smem& sm) {
         t = tn;
         // prop!(ks[1], t, tn) with the operator at tn; each stage then
         // re-evaluates it at its own t2
-        zg_refresh(in, sm, t, rho, kfac);
-        if (h0 != 0.0) {
-            double2* K0 = K[0];
-            for (int k = fresh_tid(); k < N; k += LH_T) K0[k] = cmul(K0[k], cexp_lh(gl(in.linop)[k], h0));
-            __syncthreads();
+        if constexpr (ZDEP) {
+            zg_refresh(in, sm, t, rho, kfac);
+            if (h0 != 0.0) {
+                double2* K0 = K[0];
+                for (int k = fresh_tid(); k < N; k += LH_T) K0[k] = cmul(K0[k], cexp_lh(gl(in.linop)[k], h0));
+                __syncthreads();
+            }
+            h0 = 0.0;
         }
-        h0 = 0.0;
 #pragma unroll 1
         for (int st = 0; st < 6 && status == LH_OK; st++) {
             double t2 = t + c_nodes[st] * dt;
             double hf = t2 - t;
-            if (st != 5) zg_refresh(in, sm, t2, rho, kfac);  // stages 5 and 6 share t + dt
+            if (ZDEP && st != 5) zg_refresh(in, sm, t2, rho, kfac);  // stages 5 and 6 share t + dt
             stage_prologue<MO, Smem>(in, sm, Y, K, st, dt, h0, hf);
             rhs_field<MO, Smem, EpiStageFO>(in, sm, EpiStageFO{K[st + 1], K[7]}, rho, kfac);
             rhs_evals++;
@@ -548,7 +555,7 @@ __device__ __forceinline__ void zdep_solve(const DInst& in, Smem& sm) {
             // GridCondition saves via dense output; ks[1] and ks[7] both hold k7
             while (saved < in.save_n && gl(in.zgrid)[saved] <= tn) {
                 double ti = gl(in.zgrid)[saved];
-                if (gl(in.saves) && ti != t && ti != tn) zg_refresh(in, sm, ti, rho, kfac);  // prop!(out, t, ti)
+                if (ZDEP && gl(in.saves) && ti != t && ti != tn) zg_refresh(in, sm, ti, rho, kfac);  // prop!(out, t, ti)
                 if (gl(in.saves)) {
                     double2* out = gl(in.saves) + (size_t)saved * N;
                     if (ti == t) {
@@ -670,19 +677,25 @@ __device__ __forceinline__ void zdep_solve(const DInst& in, Smem& sm) {
     __syncthreads();
 }
 
-
-template <int MO, int MC>
-__global__ __launch_bounds__(LH_T) void lh_zdep_solve(const DInst* insts, const double2* __restrict__ twg) {
+template <int MO, int MC, bool ZDEP>
+__global__ __launch_bounds__(LH_T) void lh_solo_solve(const DInst* insts, const double2* __restrict__ twg) {
     __shared__ SmemT<MO> sm;
     tw_load(sm.tw, twg);
     __syncthreads();
-    zdep_solve<MO, MC, SmemT<MO>>(insts[blockIdx.x], sm);
+    solo_solve<MO, MC, ZDEP, SmemT<MO>>(insts[blockIdx.x], sm);
 }
 
-void launch_zdep(int cls, int n, const DInst* dinst, const double2* tw, hipStream_t s) {
+template <bool ZDEP>
+static void launch(int cls, int n, const DInst* d, const double2* tw, hipStream_t s) {
     switch (cls) {
-        case LH_CLASS_16384: hipLaunchKernelGGL((lh_zdep_solve<8192, 4096>), dim3(n), dim3(LH_T), 0, s, dinst, tw); break;
-        case LH_CLASS_8192: hipLaunchKernelGGL((lh_zdep_solve<4096, 2048>), dim3(n), dim3(LH_T), 0, s, dinst, tw); break;
-        default: hipLaunchKernelGGL((lh_zdep_solve<2048, 1024>), dim3(n), dim3(LH_T), 0, s, dinst, tw); break;
+        case LH_CLASS_16384: hipLaunchKernelGGL((lh_solo_solve<8192, 4096, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
+        case LH_CLASS_8192: hipLaunchKernelGGL((lh_solo_solve<4096, 2048, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
+        default: hipLaunchKernelGGL((lh_solo_solve<2048, 1024, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
     }
+}
+void launch_solo(int cls, int n, const DInst* d, const double2* tw, hipStream_t s, bool zdep) {
+    if (zdep)
+        launch<true>(cls, n, d, tw, s);
+    else
+        launch<false>(cls, n, d, tw, s);
 }
