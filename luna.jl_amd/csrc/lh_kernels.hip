@@ -699,13 +699,14 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
 // Whether the constant-fill field instances of a batch run on one workgroup each
 // (lh_solo.hip) instead of on gangs.  Both ways are priced with the estimated
 // lengths of their runs: alone, the slowest instance or the work over the CUs
-// decides; on gangs the work does.  µs per right-hand side: one workgroup 23.4,
-// 37.4, 63.7 at Nto = 4096, 8192, 16384; gangs, per instance on the whole chip,
-// 0.275, 0.31, 0.455 at one workgroup per CU and 0.241, 0.26, 0.382 on dense
-// kernels.  256 equal instances: 3.8, 6.1, 10.4 ms alone against 10.1, 10.9, 16.0
-// on gangs; a sweep of 256 whose lengths spread by a factor of ten (mean half the
-// longest): 51 against 40.  The rule depends on the batch alone, so a batch gives
-// the same bits every time; the two ways agree to rounding.
+// decides; on gangs the work does, and a tail of a tenth or more.  µs per
+// right-hand side: one workgroup 23.4, 37.4, 63.7 at Nto = 4096, 8192, 16384;
+// gangs, per instance on the whole chip, 0.275, 0.31, 0.455 at one workgroup per
+// CU and 0.241, 0.26, 0.382 on dense kernels.  256 equal instances: 3.8, 6.1,
+// 10.4 ms alone against 10.1, 10.9, 16.0 on gangs; sweeps whose longest run is
+// twice the mean: 51 against 40 ms with 256 points, 26 against 34 with 384 (half
+// as long), 53 against 76 with 512.  The rule depends on the batch alone, so a
+// batch gives the same bits every time; the two ways agree to rounding.
 static bool solo_class(const lh_ctx* c) {
     const int cls = ctx_class(c);
     return c->d.transform == LH_TRANS_MODEAVG && !c->zg_on && !c->d.raman &&
@@ -733,7 +734,7 @@ static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
                                 : (cls == LH_CLASS_16384 ? 0.455 : cls == LH_CLASS_8192 ? 0.31 : 0.275));
         }
     }
-    return m > 0 && std::max(longest, alone) < gangs;
+    return m > 0 && std::max(longest, alone) < 1.1 * gangs;
 }
 
 static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, DInst* in, lh_stats* dstats_slot,
@@ -1469,7 +1470,7 @@ int lh_get_saves(lh_ctx* c, double* saves, double* zsaves) {
 // One stream per (device, size class and kernel) for the batched launches, created on
 // first use and kept for the process (default priority).
 static std::mutex g_cls_mu;
-static hipStream_t g_cls_stream[64][4 * LH_NCLASS];
+static hipStream_t g_cls_stream[64][3 * LH_NCLASS];
 
 static int class_stream(int dev, int c, hipStream_t* out) {
     if (dev < 0 || dev >= 64) return LH_E_ARG;
@@ -1584,7 +1585,9 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         const int cls = order[gi / N_VAR], var = gi % N_VAR, c = var * LH_NCLASS + cls;
         if (!count[c]) continue;
         hipStream_t cs;
-        if (class_stream(dev, c, &cs) != LH_OK || hipEventCreateWithFlags(&done[c], hipEventDisableTiming) != hipSuccess ||
+        // a class is on gangs or alone, never both: one stream, so the classes'
+        // launches keep the hardware queues that let them run side by side
+        if (class_stream(dev, var == V_SOLO ? cls : c, &cs) != LH_OK || hipEventCreateWithFlags(&done[c], hipEventDisableTiming) != hipSuccess ||
             hipStreamWaitEvent(cs, ready, 0) != hipSuccess || hipEventCreate(&t0[c]) != hipSuccess ||
             hipEventCreate(&t1[c]) != hipSuccess || hipEventRecord(t0[c], cs) != hipSuccess) {
             st = LH_E_HIP;
