@@ -217,8 +217,8 @@ int lh_solve_stream(lh_ctx *ctx, double *Ew_inout, const lh_rk_opts *opts, lh_ou
 
 /* Batched solve: n independent instances (each its own grid, constants, step
  * size control and status) in one persistent launch per grid class, a gang of
- * four workgroups per instance (z-dependent fills and large even batches of
- * field grids: one workgroup, whose results agree with a gang's to rounding),
+ * four workgroups per instance (z-dependent fills and large even batches:
+ * one workgroup, whose results agree with a gang's to rounding),
  * the expensive instances first.  Radial contexts (whose one instance fills the GPU)
  * are solved one after another by a graph-replayed per-step launch sequence.
  * Replaces the per-point loop of Scans.runscan src/Scans.jl:275-430.

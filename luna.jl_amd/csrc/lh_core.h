@@ -427,8 +427,10 @@ __device__ __forceinline__ double field_at(const Smem& sm, int g, double e_scale
 // The series is processed in rounds of QR samples per thread (contiguous
 // chunks), with the three cumtrapz integrals carried from round to round;
 // each thread's samples are touched only by that thread.
-template <int MO, class Smem>
-__device__ __forceinline__ void pointwise_field(const DInst& in, Smem& sm, double rho, double kfac) {
+// RAMAN: praman holds P(t) of the Raman response, packed pairs.
+template <int MO, class Smem, bool RAMAN = false>
+__device__ __forceinline__ void pointwise_field(const DInst& in, Smem& sm, double rho, double kfac,
+                                                const double2* praman = nullptr) {
     constexpr int QT = 2 * MO / LH_T;          // samples per thread over all rounds
     constexpr int QR = (QT > 16) ? 16 : QT;    // samples per thread per round
     constexpr int NR = QT / QR;                // rounds
@@ -555,6 +557,11 @@ __device__ __forceinline__ void pointwise_field(const DInst& in, Smem& sm, doubl
             if (plasma) {
                 p0 = p0 + rho * a[2 * s2];
                 p1 = p1 + rho * a[2 * s2 + 1];
+            }
+            if constexpr (RAMAN) {  // RamanPolarField: Pout = ρ·E·P (src/Nonlinear.jl:323-325)
+                const double2 pr = gl(praman)[g >> 1];
+                p0 = p0 + (rho * E0) * pr.x;
+                p1 = p1 + (rho * E1) * pr.y;
             }
             sm.buf[pad(g >> 1)] = make_double2(p0 * tw[g], p1 * tw[g + 1]);
         }

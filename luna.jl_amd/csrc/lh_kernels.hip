@@ -696,42 +696,55 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
     return isfinite(x) ? x * class_us(ctx_class(c)) : 0.0;
 }
 
-// Whether the constant-fill field instances of a batch run on one workgroup each
+// Whether the constant-fill instances of a batch run on one workgroup each
 // (lh_solo.hip) instead of on gangs.  Both ways are priced with the estimated
 // lengths of their runs: alone, the slowest instance or the work over the CUs
 // decides; on gangs the work does, and a tail of a tenth or more.  µs per
 // right-hand side: one workgroup 23.4, 37.4, 63.7 at Nto = 4096, 8192, 16384;
 // gangs, per instance on the whole chip, 0.275, 0.31, 0.455 at one workgroup per
-// CU and 0.241, 0.26, 0.382 on dense kernels.  256 equal instances: 3.8, 6.1,
+// CU and 0.241, 0.26, 0.382 on dense kernels; the other entries of solo_price
+// likewise (with a Raman response; the envelope grid of 4096 points).  Grids that
+// have no entry are faster on gangs at every number of instances.  256 equal instances: 3.8, 6.1,
 // 10.4 ms alone against 10.1, 10.9, 16.0 on gangs; sweeps whose longest run is
 // twice the mean: 51 against 40 ms with 256 points, 26 against 34 with 384 (half
 // as long), 53 against 76 with 512.  The rule depends on the batch alone, so a
 // batch gives the same bits every time; the two ways agree to rounding.
-static bool solo_class(const lh_ctx* c) {
+struct SoloPrice {
+    double alone, gang, dense;  // µs: alone per right-hand side, on gangs per instance
+};
+static bool solo_price(const lh_ctx* c, SoloPrice* p) {
+    if (c->d.transform != LH_TRANS_MODEAVG || c->zg_on) return false;
     const int cls = ctx_class(c);
-    return c->d.transform == LH_TRANS_MODEAVG && !c->zg_on && !c->d.raman &&
-           (cls == LH_CLASS_16384 || cls == LH_CLASS_8192 || cls == LH_CLASS_4096);
+    if (cls == LH_CLASS_ENV4096) return *p = {57.5, 0.341, 0.341}, true;
+    if (c->d.grid_kind != LH_GRID_REAL) return false;
+    if (c->d.raman) {
+        if (cls == LH_CLASS_8192) return *p = {103.7, 0.511, 0.511}, true;
+        if (cls == LH_CLASS_4096) return *p = {48.4, 0.404, 0.404}, true;
+        return false;
+    }
+    if (cls == LH_CLASS_16384) return *p = {63.7, 0.455, 0.382}, true;
+    if (cls == LH_CLASS_8192) return *p = {37.4, 0.31, 0.26}, true;
+    if (cls == LH_CLASS_4096) return *p = {23.4, 0.275, 0.241}, true;
+    return false;
 }
 static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
     const bool dense = n > LG_DENSE_ABOVE;
     double longest = 0.0, alone = 0.0, gangs = 0.0;
     int m = 0, zero = 0;
+    SoloPrice p;
     for (int pass = 0; pass < 2; pass++) {
         for (int i = 0; i < n; i++) {
-            if (!solo_class(ctxs[i])) continue;
-            const int cls = ctx_class(ctxs[i]);
-            double w = solve_cost(ctxs[i], op[i]) / class_us(cls);
+            if (!solo_price(ctxs[i], &p)) continue;
+            double w = solve_cost(ctxs[i], op[i]) / class_us(ctx_class(ctxs[i]));
             if (pass == 0) {
                 m++;
                 zero += (w == 0.0);
                 continue;
             }
             if (zero == m) w = 1.0;  // linear runs: equal lengths
-            const double us = cls == LH_CLASS_16384 ? 63.7 : cls == LH_CLASS_8192 ? 37.4 : 23.4;
-            longest = std::max(longest, w * us);
-            alone += w * us / LG_MAX_WG;
-            gangs += w * (dense ? (cls == LH_CLASS_16384 ? 0.382 : cls == LH_CLASS_8192 ? 0.26 : 0.241)
-                                : (cls == LH_CLASS_16384 ? 0.455 : cls == LH_CLASS_8192 ? 0.31 : 0.275));
+            longest = std::max(longest, w * p.alone);
+            alone += w * p.alone / LG_MAX_WG;
+            gangs += w * (dense ? p.dense : p.gang);
         }
     }
     return m > 0 && std::max(longest, alone) < 1.1 * gangs;
@@ -1508,18 +1521,21 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     // follow as those run out of jobs.  Radial contexts block the host and come
     // last.
     const bool solo = solo_pays(ctxs, op, n);
-    enum { V_GANG, V_RAMAN, V_ZDEP, V_SOLO, N_VAR };
+    enum { V_GANG, V_RAMAN, V_ZDEP, V_SOLO, V_SOLOR, N_VAR };
     constexpr int NG = N_VAR * LH_NCLASS;
     static const int order[LH_NCLASS] = {LH_CLASS_32768, LH_CLASS_ENV16384, LH_CLASS_16384, LH_CLASS_ENV8192,
                                          LH_CLASS_8192,  LH_CLASS_ENV4096,  LH_CLASS_4096,  LH_CLASS_RADIAL};
     auto group_of = [&](const lh_ctx* c) {
         const bool fr = c->d.transform == LH_TRANS_MODEAVG && c->d.grid_kind == LH_GRID_REAL && c->d.raman;
-        return (c->zg_on ? V_ZDEP : fr ? V_RAMAN : (solo && solo_class(c)) ? V_SOLO : V_GANG) * LH_NCLASS + ctx_class(c);
+        SoloPrice p;
+        const bool one = solo && solo_price(c, &p);
+        return (c->zg_on ? V_ZDEP : fr ? (one ? V_SOLOR : V_RAMAN) : (one ? V_SOLO : V_GANG)) * LH_NCLASS + ctx_class(c);
     };
     int count[NG] = {0}, first[NG] = {0};
     for (int i = 0; i < n; i++) count[group_of(ctxs[i])]++;
     for (int c = 0; c < LH_NCLASS; c++)  // refused as before: both in one class
-        if (count[V_RAMAN * LH_NCLASS + c] && count[V_ZDEP * LH_NCLASS + c]) return LH_E_ARG;
+        if ((count[V_RAMAN * LH_NCLASS + c] || count[V_SOLOR * LH_NCLASS + c]) && count[V_ZDEP * LH_NCLASS + c])
+            return LH_E_ARG;
     for (int c = 1; c < NG; c++) first[c] = first[c - 1] + count[c - 1];
     // Within a group the expensive instances come first (the gangs take them in
     // order), so the last ones to run are short: a 256-point sweep ends 10 ms
@@ -1587,7 +1603,7 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         hipStream_t cs;
         // a class is on gangs or alone, never both: one stream, so the classes'
         // launches keep the hardware queues that let them run side by side
-        if (class_stream(dev, var == V_SOLO ? cls : c, &cs) != LH_OK || hipEventCreateWithFlags(&done[c], hipEventDisableTiming) != hipSuccess ||
+        if (class_stream(dev, var == V_SOLO ? cls : var == V_SOLOR ? V_RAMAN * LH_NCLASS + cls : c, &cs) != LH_OK || hipEventCreateWithFlags(&done[c], hipEventDisableTiming) != hipSuccess ||
             hipStreamWaitEvent(cs, ready, 0) != hipSuccess || hipEventCreate(&t0[c]) != hipSuccess ||
             hipEventCreate(&t1[c]) != hipSuccess || hipEventRecord(t0[c], cs) != hipSuccess) {
             st = LH_E_HIP;
@@ -1599,8 +1615,8 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
                 if (ctx_class(ctxs[i]) == LH_CLASS_RADIAL)
                     st = rad_solve(ctxs[i], op[i], want_saves != 0, cs, &rad_stats[i]);
             if (st) break;
-        } else if (var == V_ZDEP || var == V_SOLO) {
-            launch_solo(cls, count[c], dinst + first[c], tw16, cs, var == V_ZDEP);
+        } else if (var >= V_ZDEP) {
+            if (!launch_solo(cls, count[c], dinst + first[c], tw16, cs, var == V_ZDEP, var == V_SOLOR)) st = LH_E_ARG;
         } else {
             const GangLaunch l{cls, nwg[c], (GangCtl*)(dblk + ctl_off[c]), dinst + first[c], tw, cs};
             if (!(dense[c] ? lg_dense_solve(l) : launch_solve(l, var == V_RAMAN, false))) st = LH_E_ARG;
@@ -2115,7 +2131,7 @@ int lh_solve_noalloc(lh_ctx* c, void* Ew_dev, const lh_rk_opts* o, void* saves_d
     }
     const GangLaunch l = launch1_of(c, base + L.inst, tw, s);
     if (c->zg_on)
-        launch_solo(cls, 1, l.d, tw16, s, true);
+        (void)launch_solo(cls, 1, l.d, tw16, s, true, false);
     else if (!launch_solve(l, c->d.raman != 0, false))
         return LH_E_ARG;
     HIPCK(hipGetLastError());

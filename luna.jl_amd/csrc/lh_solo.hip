@@ -1,4 +1,4 @@
-// lh_solo.hip -- propagation on a field grid, one workgroup per instance (gfx950).
+// lh_solo.hip -- propagation with one workgroup per instance (gfx950).
 //
 // Two kinds of instances run here instead of on gangs of workgroups (lh_gang.h).
 //
@@ -9,7 +9,7 @@
 // operations in the right-hand side shifts the step positions z by a relative
 // 1e-13 through the error estimate, which is enough to flip such a unit at some
 // z: the same solver on gangs took 19.4 ms instead of 42.6 for a 0.5 m
-// propagation at Nto = 16384, but landed 5e-8 away.
+// propagation at Nto = 16384, but landed 5e-8 away.  Field grids only.
 //
 // Large even batches: a gang exchanges its series through the L2 and waits at
 // barriers, a workgroup alone does neither, so with an instance for every CU and
@@ -54,13 +54,138 @@ struct EpiStageFO {
     }
 };
 
+// exp(−2πi k/L) for the zero-padded Raman transforms: L up to LH_TWN from
+// the table; L = 2·LH_TWN gives even k from the table and odd k one more
+// factor exp(−2πi/L).
+template <int L>
+__device__ __forceinline__ double2 tw_frac(const TwLds& tw, int k) {
+    if constexpr (L <= LH_TWN) {
+        return tw_get(tw, k * (LH_TWN / L));
+    } else {
+        static_assert(L == 2 * LH_TWN, "tw_frac: L up to 2·LH_TWN");
+        double2 w = tw_get(tw, k >> 1);
+        if (k & 1) {
+            double sn, cs;
+            sincos(-6.283185307179586476925286766559 / (double)L, &sn, &cs);
+            w = cmul(w, make_double2(cs, sn));
+        }
+        return w;
+    }
+}
+
+// Unnormalised complex FFT of NO = 2·M points held in HBM (natural order, in
+// place in g); tmp: M points of HBM.  X[k] = E[k] + w^k O[k], X[k+M] =
+// E[k] − w^k O[k], with E, O the transforms of the even and odd samples and
+// w = exp(∓2πi/NO).  Starts and ends with a workgroup barrier.
+template <int M, bool INV, class Smem>
+__device__ __forceinline__ void fft_big(double2* g, double2* tmp, Smem& sm) {
+    const int tid = fresh_tid();
+    __syncthreads();
+    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j];
+    __syncthreads();
+    fft_lds<M, INV>(sm.buf, sm.tw);
+    for (int j = tid; j < M; j += LH_T) tmp[j] = sm.buf[pad(j)];
+    __syncthreads();
+    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j + 1];
+    __syncthreads();
+    fft_lds<M, INV>(sm.buf, sm.tw);
+    constexpr int TS = LH_TWN / (2 * M);
+    for (int k = tid; k < M; k += LH_T) {
+        double2 w = tw_get(sm.tw, k * TS);
+        if (INV) w.y = -w.y;
+        const double2 o = cmul(w, sm.buf[pad(k)]), e = tmp[k];
+        g[k] = cadd(e, o);
+        g[k + M] = csub(e, o);
+    }
+    __syncthreads();
+}
+
+// r2c post-step of a 2·NO-point real transform whose packed NO-point
+// transform Z is in HBM: X[k] = E + w^k O (as r2c_bin).
+template <int NO, class Smem>
+__device__ __forceinline__ double2 r2c_bin_big(const double2* Z, const Smem& sm, int k) {
+    double2 zk = Z[k == NO ? 0 : k];
+    double2 zc = cconj(Z[k == 0 ? 0 : NO - k]);
+    double2 E = cscal(0.5, cadd(zk, zc));
+    double2 d = csub(zk, zc);
+    double2 O = make_double2(0.5 * d.y, -(0.5 * d.x));
+    double2 w = (k == NO) ? make_double2(-1.0, 0.0) : tw_frac<2 * NO>(sm.tw, k);
+    return cadd(E, cmul(w, O));
+}
+
+// The convolution step of the zero-padded Raman transform (2·NO reals packed
+// into the NO-point transform Z in HBM): r2c post-step, ×hω·δt, and the c2r
+// pre-pack of the product, pairwise (k, NO − k) in place.
+template <int NO, class Smem>
+__device__ __forceinline__ void raman_spectrum_big(const DInst& in, const Smem& sm, double2* W) {
+    const int tid = fresh_tid();
+    for (int k = tid; k <= NO / 2; k += LH_T) {
+        const int m = NO - k;
+        if (k == 0) {
+            double2 Y0 = cmul(gl(in.hwdt)[0], r2c_bin_big<NO>(W, sm, 0));
+            double2 YM = cmul(gl(in.hwdt)[NO], r2c_bin_big<NO>(W, sm, NO));
+            Y0.y = 0.0;
+            YM.y = 0.0;
+            const double2 A = cadd(Y0, cconj(YM)), B = csub(Y0, cconj(YM));
+            W[0] = cadd(A, cmul_pi(B));
+        } else if (k == NO / 2) {
+            const double2 Yk = cmul(gl(in.hwdt)[k], r2c_bin_big<NO>(W, sm, k));
+            const double2 A = cadd(Yk, cconj(Yk));
+            const double2 B = cmul(csub(Yk, cconj(Yk)), cconj(tw_frac<2 * NO>(sm.tw, k)));
+            W[k] = cadd(A, cmul_pi(B));
+        } else {
+            const double2 Yk = cmul(gl(in.hwdt)[k], r2c_bin_big<NO>(W, sm, k));
+            const double2 Ym = cmul(gl(in.hwdt)[m], r2c_bin_big<NO>(W, sm, m));
+            const double2 wk = cconj(tw_frac<2 * NO>(sm.tw, k)), wm = cconj(tw_frac<2 * NO>(sm.tw, m));
+            const double2 Ak = cadd(Yk, cconj(Ym)), Bk = cmul(csub(Yk, cconj(Ym)), wk);
+            const double2 Am = cadd(Ym, cconj(Yk)), Bm = cmul(csub(Ym, cconj(Yk)), wm);
+            W[k] = cadd(Ak, cmul_pi(Bk));
+            W[m] = cadd(Am, cmul_pi(Bm));
+        }
+    }
+}
+
+// RamanPolarField with third-harmonic terms (src/Nonlinear.jl:183-247,
+// 284-333, thg = true) for a series of Nto = 2·MO reals held packed in LDS
+// (before the e_scale factor).  E² over the zero-padded 2·Nto reals is one
+// 2·MO-point complex transform, run through HBM as two MO-point LDS transforms
+// (fft_big); ×hω·δt; back; P(t) lands in the last MO points of the exchange area
+// (4·MO) as packed pairs.  The LDS series is restored from its copy in the first.
+template <int MO, class Smem>
+__device__ __forceinline__ void raman_field(const DInst& in, Smem& sm) {
+    constexpr int NR = 2 * MO;
+    double2* S = gl(in.gx);
+    double2* W = gl(in.gx) + MO;
+    double2* T = gl(in.gx) + 3 * MO;
+    const int tid = fresh_tid();
+    const double es = in.e_scale;
+    for (int j = tid; j < MO; j += LH_T) {
+        const double2 z = sm.buf[pad(j)];
+        const double e0 = z.x * es, e1 = z.y * es;
+        S[j] = z;
+        W[j] = make_double2(e0 * e0, e1 * e1);  // E² (thg: E.^2), reals packed in pairs
+        W[j + MO] = make_double2(0.0, 0.0);     // zero padding to 2·Nto reals
+    }
+    fft_big<MO, false>(W, T, sm);
+    raman_spectrum_big<NR>(in, sm, W);
+    fft_big<MO, true>(W, T, sm);
+    const double inv2n = in.inv_2n;
+    for (int j = tid; j < MO; j += LH_T) {
+        const double2 p = W[j];
+        T[j] = make_double2(p.x * inv2n, p.y * inv2n);
+        sm.buf[pad(j)] = S[j];
+    }
+    __syncthreads();
+}
+
 // Field-grid mode-averaged transform on LDS data.  On entry buf holds the c2r
 // pre-pack of sc_t·Eω.  Hands the output bins k < N to epi.
-template <int MO, class Smem, class Epi>
+template <int MO, bool RAMAN, class Smem, class Epi>
 __device__ __forceinline__ void rhs_field(const DInst& in, Smem& sm, Epi epi, double rho, double kfac) {
     __syncthreads();
     fft_lds<MO, true>(sm.buf, sm.tw);
-    pointwise_field<MO, Smem>(in, sm, rho, kfac);
+    if constexpr (RAMAN) raman_field<MO, Smem>(in, sm);
+    pointwise_field<MO, Smem, RAMAN>(in, sm, rho, kfac, RAMAN ? in.gx + 3 * MO : nullptr);
     constexpr int N = Bins<MO>::N, NPT = Bins<MO>::NPT;
     static_assert(NPT <= 9, "one epilogue chunk");
     double2 res[NPT];
@@ -370,10 +495,255 @@ __device__ __forceinline__ void stats_time(const DInst& in, Smem& sm, double s0,
     __syncthreads();
 }
 
+// Envelope grid of NO points (Nto = Nt).
+template <int NO, class Smem>
+__device__ __forceinline__ void stage_prologue_env(const DInst& in, Smem& sm, const double2* Y, const KSet& K,
+                                                   int stage, double dt, double h0, double hf) {
+    constexpr int N = NO, NPT = NO / LH_T;
+    const int tid = fresh_tid();
+    double2 yb[NPT], L[NPT];
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        int k = tid + i * LH_T;
+        bool v = k < N;
+        yb[i] = v ? Y[k] : make_double2(0.0, 0.0);
+        L[i] = v ? static_cast<const double2*>(gl(in.linop))[k] : make_double2(0.0, 0.0);
+    }
+    if (stage == 0 && h0 != 0.0) {
+        double2* K0 = K[0];
+        constexpr int CH = (NPT > 9) ? 8 : NPT;  // a chunk's loads before its first store
+        static_assert(NPT % CH == 0, "prologue chunks");
+#pragma unroll
+        for (int c = 0; c < NPT; c += CH) {
+            double2 kv[CH];
+#pragma unroll
+            for (int i = 0; i < CH; i++) {
+                int k = tid + (c + i) * LH_T;
+                kv[i] = (k < N) ? K0[k] : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int i = 0; i < CH; i++) {
+                int k = tid + (c + i) * LH_T;
+                if (k < N) K0[k] = cmul(kv[i], cexp_lh(L[c + i], h0));
+            }
+        }
+    }
+#pragma unroll 1
+    for (int j = 0; j <= stage; j++) {
+        const double cj = dt * c_B[stage][j];
+        if (cj == 0.0) continue;
+        const double2* Kj = K[j];
+#pragma unroll
+        for (int i = 0; i < NPT; i++) {
+            int k = tid + i * LH_T;
+            if (k < N) yb[i] = cadd(yb[i], cscal(cj, Kj[k]));
+        }
+    }
+    const double sc_t = in.sc_t;
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        int k = tid + i * LH_T;
+        if (k < N) {
+            // exp(L·hf), and for the stage epilogue exp(L·(t − t2)) = exp(−L·hf)
+            // from the same exp and sincos into slot 7 (saves the envelope
+            // epilogue, with 16 bins per thread, its own transcendental pass)
+            double2 yp = yb[i], inv = make_double2(1.0, 0.0);
+            if (hf != 0.0) yp = cmul(yb[i], cexp_lh_inv(L[i], hf, inv));
+            sm.buf[pad(k)] = cscal(sc_t, yp);
+            K[7][k] = inv;
+        }
+    }
+}
+
+// TransModeAvg on an envelope grid with Kerr_env and RamanPolarEnv
+// (src/NonlinearRHS.jl:25-32, 47-53, 362-373, 389-399; src/Nonlinear.jl:47-49,
+// 63-73, 282-333).  The Raman convolution of ½|E|² with h(t) over the
+// zero-padded 2·Nto grid is done as a real transform: r2c of 2·Nto reals (a
+// length-Nto complex FFT), ×(hω δt), c2r, with E(t) in the exchange area meanwhile.
+template <int NO, class Smem, class Epi>
+__device__ __forceinline__ void rhs_env(const DInst& in, Smem& sm, Epi epi) {
+    constexpr int PER = NO / LH_T;  // complex samples per thread (contiguous chunk)
+    const int tid = fresh_tid();
+    const int i0 = PER * tid;
+    __syncthreads();
+    fft_lds<NO, true>(sm.buf, sm.tw);
+    const double es = in.e_scale;
+    if (in.raman) {
+        double2 E[PER];
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            double2 z = sm.buf[pad(i0 + q)];
+            E[q] = make_double2(z.x * es, z.y * es);
+            gl(in.gx)[i0 + q] = E[q];
+        }
+        __syncthreads();  // every thread has read its E before the packing overwrites
+#pragma unroll
+        for (int q = 0; q < PER / 2; q++) {
+            double a0 = 0.5 * (E[2 * q].x * E[2 * q].x + E[2 * q].y * E[2 * q].y);
+            double a1 = 0.5 * (E[2 * q + 1].x * E[2 * q + 1].x + E[2 * q + 1].y * E[2 * q + 1].y);
+            sm.buf[pad(i0 / 2 + q)] = make_double2(a0, a1);        // ½|E|², reals packed in pairs
+            sm.buf[pad(NO / 2 + i0 / 2 + q)] = make_double2(0.0, 0.0);  // zero padding to 2·Nto
+        }
+        __syncthreads();
+        fft_lds<NO, false>(sm.buf, sm.tw);
+        // r2c post-step of the 2·Nto-point transform, ×hω·δt, and the c2r
+        // pre-pack of the product, pairwise (k, Nto-k) in place
+        constexpr int TS = LH_TWN / (2 * NO);
+        for (int k = tid; k <= NO / 2; k += LH_T) {
+            int m = NO - k;
+            if (k == 0) {
+                double2 Y0 = cmul(gl(in.hwdt)[0], r2c_bin<NO>(sm.buf, sm.tw, 0));
+                double2 YM = cmul(gl(in.hwdt)[NO], r2c_bin<NO>(sm.buf, sm.tw, NO));
+                Y0.y = 0.0;
+                YM.y = 0.0;
+                double2 A = cadd(Y0, cconj(YM)), B = csub(Y0, cconj(YM));
+                sm.buf[pad(0)] = cadd(A, cmul_pi(B));
+            } else if (k == NO / 2) {
+                double2 Yk = cmul(gl(in.hwdt)[k], r2c_bin<NO>(sm.buf, sm.tw, k));
+                double2 A = cadd(Yk, cconj(Yk));
+                double2 B = cmul(csub(Yk, cconj(Yk)), cconj(tw_get(sm.tw, k * TS)));
+                sm.buf[pad(k)] = cadd(A, cmul_pi(B));
+            } else {
+                double2 Yk = cmul(gl(in.hwdt)[k], r2c_bin<NO>(sm.buf, sm.tw, k));
+                double2 Ym = cmul(gl(in.hwdt)[m], r2c_bin<NO>(sm.buf, sm.tw, m));
+                double2 wk = cconj(tw_get(sm.tw, k * TS)), wm = cconj(tw_get(sm.tw, m * TS));
+                double2 Ak = cadd(Yk, cconj(Ym)), Bk = cmul(csub(Yk, cconj(Ym)), wk);
+                double2 Am = cadd(Ym, cconj(Yk)), Bm = cmul(csub(Ym, cconj(Yk)), wm);
+                sm.buf[pad(k)] = cadd(Ak, cmul_pi(Bk));
+                sm.buf[pad(m)] = cadd(Am, cmul_pi(Bm));
+            }
+        }
+        __syncthreads();
+        fft_lds<NO, true>(sm.buf, sm.tw);  // P(t) on the 2·Nto grid, packed in pairs
+        double P[PER];
+#pragma unroll
+        for (int q = 0; q < PER / 2; q++) {
+            double2 z = sm.buf[pad(i0 / 2 + q)];
+            P[2 * q] = z.x * in.inv_2n;
+            P[2 * q + 1] = z.y * in.inv_2n;
+        }
+        __syncthreads();
+        const double rho = in.density, k34 = in.kerr34;
+        const bool kerr = (in.kerr == LH_KERR_ENV);
+        const double* tw = gl(in.to_win);
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            double2 e = gl(in.gx)[i0 + q];
+            double2 p = make_double2(0.0, 0.0);
+            if (kerr) {
+                double s = k34 * (e.x * e.x + e.y * e.y);
+                p = make_double2(s * e.x, s * e.y);
+            }
+            double2 re = make_double2(rho * e.x, rho * e.y);
+            p = cadd(p, make_double2(re.x * P[q], re.y * P[q]));
+            sm.buf[pad(i0 + q)] = make_double2(p.x * tw[i0 + q], p.y * tw[i0 + q]);
+        }
+    } else {
+        const double k34 = in.kerr34;
+        const bool kerr = (in.kerr == LH_KERR_ENV);
+        const double* tw = gl(in.to_win);
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            double2 z = sm.buf[pad(i0 + q)];
+            double2 e = make_double2(z.x * es, z.y * es);
+            double2 p = make_double2(0.0, 0.0);
+            if (kerr) {
+                double s = k34 * (e.x * e.x + e.y * e.y);
+                p = make_double2(s * e.x, s * e.y);
+            }
+            sm.buf[pad(i0 + q)] = make_double2(p.x * tw[i0 + q], p.y * tw[i0 + q]);
+        }
+    }
+    constexpr int N = NO, NPT = NO / LH_T;
+    double2 of[NPT];
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        int k = tid + i * LH_T;
+        of[i] = (k < N) ? static_cast<const double2*>(gl(in.outfac))[k] : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    fft_lds<NO, false>(sm.buf, sm.tw);
+    constexpr int CH = NPT;
+    static_assert(NPT <= 9, "one epilogue chunk");
+#pragma unroll
+    for (int c = 0; c < NPT; c += CH) {
+        double2 res[CH];
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            int k = tid + (c + i) * LH_T;
+            res[i] = (k < N) ? cmul(sm.buf[pad(k)], of[c + i]) : make_double2(0.0, 0.0);
+        }
+        epi(res, N);
+    }
+}
+
+// stepfun on the envelope grid (src/Luna.jl:366-370 with a c2c FT).
+template <int NT, class Smem>
+__device__ __forceinline__ void stepfun_env(const DInst& in, Smem& sm, double2* YN, double h, double* rec, double z,
+                                            double dz, double rho) {
+    constexpr int NPT = (NT + LH_T - 1) / LH_T;
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        int k = fresh_tid() + i * LH_T;
+        if (k < NT) {
+            double2 v = YN[k];
+            if (h != 0.0) v = cmul(v, cexp_lh(gl(in.linop)[k], h));
+            sm.buf[pad(k)] = cscal(gl(in.omega_win)[k], v);
+        }
+    }
+    __syncthreads();
+    fft_lds<NT, true>(sm.buf, sm.tw);
+    const double inv_nt = in.inv_nt;
+    for (int j = fresh_tid(); j < NT; j += LH_T) {
+        double2 z = sm.buf[pad(j)];
+        double w = gl(in.t_win)[j];
+        sm.buf[pad(j)] = make_double2((inv_nt * z.x) * w, (inv_nt * z.y) * w);
+    }
+    __syncthreads();
+    fft_lds<NT, false>(sm.buf, sm.tw);
+    double s0 = 0.0, s1 = 0.0, se = 0.0;
+    WinSums ws = {{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        int k = fresh_tid() + i * LH_T;
+        if (k < NT) {
+            double2 v = sm.buf[pad(k)];
+            YN[k] = v;
+            if (rec) {  // the envelope's analytic field is ifft(Eω): the spectrum stays in place
+                double a = v.x * v.x + v.y * v.y;
+                s0 += a;
+                s1 += gl(in.st_omega)[k] * a;
+                se += gl(in.st_ew)[k] * a;
+                win_add(in, ws, k, a);
+            }
+        }
+    }
+    if (rec)
+        stats_time<1, NT, Smem>(in, sm, s0, s1, se, ws, z, dz, rho, rec);
+    else
+        __syncthreads();
+}
+
+template <int KIND, int MO, class Smem>
+__device__ __forceinline__ void prologue(const DInst& in, Smem& sm, const double2* Y, const KSet& K, int stage, double dt,
+                                         double h0, double hf) {
+    if constexpr (KIND == 0)
+        stage_prologue<MO, Smem>(in, sm, Y, K, stage, dt, h0, hf);
+    else
+        stage_prologue_env<MO, Smem>(in, sm, Y, K, stage, dt, h0, hf);
+}
+template <int KIND, int MO, bool RAMAN, class Smem, class Epi>
+__device__ __forceinline__ void rhs(const DInst& in, Smem& sm, Epi epi, double rho, double kfac) {
+    if constexpr (KIND == 0)
+        rhs_field<MO, RAMAN, Smem, Epi>(in, sm, epi, rho, kfac);
+    else
+        rhs_env<MO, Smem>(in, sm, epi);
+}
+
 // Adaptive solve of one instance (Luna.run → RK45.solve_precon).
-template <int MO, int MC, bool ZDEP, class Smem>
+template <int KIND, int MO, int MC, bool ZDEP, bool RAMAN, class Smem>
 __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
-    constexpr int N = Bins<MO>::N, NPT = Bins<MO>::NPT;
+    constexpr int N = (KIND == 0) ? Bins<MO>::N : MO, NPT = (N + LH_T - 1) / LH_T;
     KSet K{gl(in.K), in.kstride, 0, 6};
     double2* const Y0 = gl(in.Y);
     double2* Y = gl(in.Y);
@@ -391,8 +761,8 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
     if constexpr (ZDEP) zg_refresh(in, sm, in.z0, rho, kfac);
 
     // PreconStepper init: k1 = fbar(y0, t, t)
-    stage_prologue<MO, Smem>(in, sm, Y, K, 0, 0.0, 0.0, 0.0);
-    rhs_field<MO, Smem, EpiStore>(in, sm, EpiStore{K[0]}, rho, kfac);
+    prologue<KIND, MO, Smem>(in, sm, Y, K, 0, 0.0, 0.0, 0.0);
+    rhs<KIND, MO, RAMAN, Smem>(in, sm, EpiStore{K[0]}, rho, kfac);
     rhs_evals++;
     __syncthreads();
     if (sm.flag != LH_OK) status = sm.flag;
@@ -422,8 +792,8 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
             double t2 = t + c_nodes[st] * dt;
             double hf = t2 - t;
             if (ZDEP && st != 5) zg_refresh(in, sm, t2, rho, kfac);  // stages 5 and 6 share t + dt
-            stage_prologue<MO, Smem>(in, sm, Y, K, st, dt, h0, hf);
-            rhs_field<MO, Smem, EpiStageFO>(in, sm, EpiStageFO{K[st + 1], K[7]}, rho, kfac);
+            prologue<KIND, MO, Smem>(in, sm, Y, K, st, dt, h0, hf);
+            rhs<KIND, MO, RAMAN, Smem>(in, sm, EpiStageFO{K[st + 1], K[7]}, rho, kfac);
             rhs_evals++;
             __syncthreads();
             if (sm.flag != LH_OK) status = sm.flag;
@@ -550,7 +920,10 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
             // (src/Output.jl:65-67) from the same LDS pass
             double* rec = (gl(in.steprec) && accepted < in.steprec_cap) ? gl(in.steprec) + (size_t)accepted * LH_NSTAT
                                                                       : nullptr;
-            stepfun_filter<MC, Smem>(in, sm, YN, tn - t, rec, tn, dtn, rho);
+            if constexpr (KIND == 0)
+                stepfun_filter<MC, Smem>(in, sm, YN, tn - t, rec, tn, dtn, rho);
+            else
+                stepfun_env<MO, Smem>(in, sm, YN, tn - t, rec, tn, dtn, rho);
             if (rec && sm.flag != LH_OK) status = sm.flag;
             // GridCondition saves via dense output; ks[1] and ks[7] both hold k7
             while (saved < in.save_n && gl(in.zgrid)[saved] <= tn) {
@@ -677,25 +1050,37 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
     __syncthreads();
 }
 
-template <int MO, int MC, bool ZDEP>
+template <int KIND, int MO, int MC, bool ZDEP, bool RAMAN>
 __global__ __launch_bounds__(LH_T) void lh_solo_solve(const DInst* insts, const double2* __restrict__ twg) {
     __shared__ SmemT<MO> sm;
     tw_load(sm.tw, twg);
     __syncthreads();
-    solo_solve<MO, MC, ZDEP, SmemT<MO>>(insts[blockIdx.x], sm);
+    solo_solve<KIND, MO, MC, ZDEP, RAMAN, SmemT<MO>>(insts[blockIdx.x], sm);
 }
 
-template <bool ZDEP>
-static void launch(int cls, int n, const DInst* d, const double2* tw, hipStream_t s) {
-    switch (cls) {
-        case LH_CLASS_16384: hipLaunchKernelGGL((lh_solo_solve<8192, 4096, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
-        case LH_CLASS_8192: hipLaunchKernelGGL((lh_solo_solve<4096, 2048, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
-        default: hipLaunchKernelGGL((lh_solo_solve<2048, 1024, ZDEP>), dim3(n), dim3(LH_T), 0, s, d, tw); break;
-    }
+template <int KIND, int MO, int MC, bool ZDEP, bool RAMAN>
+static void launch(int n, const DInst* d, const double2* tw, hipStream_t s) {
+    hipLaunchKernelGGL((lh_solo_solve<KIND, MO, MC, ZDEP, RAMAN>), dim3(n), dim3(LH_T), 0, s, d, tw);
 }
-void launch_solo(int cls, int n, const DInst* d, const double2* tw, hipStream_t s, bool zdep) {
-    if (zdep)
-        launch<true>(cls, n, d, tw, s);
-    else
-        launch<false>(cls, n, d, tw, s);
+bool launch_solo(int cls, int n, const DInst* d, const double2* tw, hipStream_t s, bool zdep, bool raman) {
+    if (cls == LH_CLASS_ENV4096) {
+        launch<1, 4096, 4096, false, false>(n, d, tw, s);
+        return true;
+    }
+    if (raman) {
+        if (cls == LH_CLASS_8192)
+            launch<0, 4096, 2048, false, true>(n, d, tw, s);
+        else if (cls == LH_CLASS_4096)
+            launch<0, 2048, 1024, false, true>(n, d, tw, s);
+        else
+            return false;
+        return true;
+    }
+    switch (cls) {
+        case LH_CLASS_16384: zdep ? launch<0, 8192, 4096, true, false>(n, d, tw, s) : launch<0, 8192, 4096, false, false>(n, d, tw, s); break;
+        case LH_CLASS_8192: zdep ? launch<0, 4096, 2048, true, false>(n, d, tw, s) : launch<0, 4096, 2048, false, false>(n, d, tw, s); break;
+        case LH_CLASS_4096: zdep ? launch<0, 2048, 1024, true, false>(n, d, tw, s) : launch<0, 2048, 1024, false, false>(n, d, tw, s); break;
+        default: return false;
+    }
+    return true;
 }
