@@ -1186,10 +1186,12 @@ int lh_rhs_device(lh_ctx* c, void* nl_dev, const void* Ew_dev, double z, void* s
         RadArgs a = rad_args(c, 1);
         a.rhs_in = (const double2*)Ew_dev;
         a.rhs_out = (double2*)nl_dev;
-        RadCtl h;
-        rad_ctl_init(&h, nullptr);
-        hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, a, h, c->rargs + 1);
-        rad_rhs_dispatch(c->rplan, c->d.grid_kind == LH_GRID_ENV, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s);
+        RadOne one;
+        one.a = a;
+        rad_ctl_init(&one.h, nullptr);
+        const bool env = c->d.grid_kind == LH_GRID_ENV;
+        if (env) hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, one.a, one.h, c->rargs + 1);
+        rad_rhs_dispatch(c->rplan, env, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s, &one);
     } else {
         DInst in = base_inst(c);
         in.rhs_in = (const double2*)Ew_dev;

@@ -100,6 +100,34 @@ __global__ __launch_bounds__(LH_T) void rad_stage_a(const RadArgs* __restrict__ 
     }
 }
 
+// The first launch of a single RHS: it brings the arguments and the control block
+// by value, works from them, and leaves them in device memory for the launches
+// that follow.
+template <int MO, int PLAN>
+__global__ __launch_bounds__(LH_T) void rad_stage_a_one(RadArgs a, RadCtl h, RadArgs* ap,
+                                                        const double2* __restrict__ twg) {
+    __shared__ SmemT<MO> sm;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *ap = a;
+        *a.ctl = h;
+    }
+    tw_load(sm.tw, twg);
+    const int c = blockIdx.x, N = a.n_omega;
+    const double2* src = gl(a.rhs_in) + (size_t)N * c;
+    for (int k = threadIdx.x; k < N; k += LH_T) sm.buf[pad(k)] = cscal(a.sc_t, src[k]);
+    for (int k = N + threadIdx.x; k <= MO; k += LH_T) sm.buf[pad(k)] = make_double2(0.0, 0.0);
+    __syncthreads();
+    c2r_prepack<MO>(sm.buf, sm.tw);
+    __syncthreads();
+    fft_lds<MO, true, PLAN>(sm.buf, sm.tw);
+    double* out = gl(a.Ek) + (size_t)a.col * c;
+    for (int j = threadIdx.x; j < MO; j += LH_T) {
+        double2 z = sm.buf[pad(j)];
+        out[2 * j] = z.x;
+        out[2 * j + 1] = z.y;
+    }
+}
+
 // ---------------------------------------------------------------- G: FP64 MFMA GEMM
 // C[M×N] = scale · A[M×K] · B[K×N]; A and C column-major (t fastest, M = Nto),
 // B[k][n] = Mt[k*Nr + n] = M[n][k].  The MFMA computes the transposed tile
@@ -525,6 +553,12 @@ __global__ void rad_step_end(const RadArgs* __restrict__ ap) {
     *ctl = s;
 }
 
+// A single RHS on the field grid carries its arguments itself (rad_stage_a_one).
+struct RadOne {
+    RadArgs a;
+    RadCtl h;
+};
+
 // Launch helpers for one RHS and one step (also used during graph capture).
 // A plan is one variant of the RHS launch sequence: the radix plan of the
 // column transforms (0: radix 8, radix 16 from 8192 points; 1: radix 16
@@ -538,9 +572,8 @@ struct RadPlan {
 static constexpr RadPlan RAD_DEFAULT_PLAN = {0, 2};
 static bool rad_plan_ok(const RadPlan& p) { return (p.fft == 0 || p.fft == 1) && (p.mt == 1 || p.mt == 2 || p.mt == 4); }
 
-// Arguments and control block of the launches that follow on the stream.  By
-// value through one launch: the two host-to-device copies it replaces took 9.6 µs
-// of a 73 µs right-hand side.
+// Arguments and control block of the launches that follow on the stream, by value
+// through one launch instead of two host-to-device copies (9.6 µs).
 __global__ __launch_bounds__(64) void rad_set(RadArgs a, RadCtl h, RadArgs* ap) {
     if (threadIdx.x != 0) return;
     *ap = a;
@@ -560,9 +593,14 @@ static int rad_tiles(const RadPlan& p, int rows, int n_r) {
 }
 
 template <int MO, int PLAN, int MT>
-static void rad_launch_rhs(const RadArgs* dargs, const double2* tw, int n_to, int n_r, int stage, hipStream_t s) {
+static void rad_launch_rhs(const RadArgs* dargs, const double2* tw, int n_to, int n_r, int stage, hipStream_t s,
+                           const RadOne* one = nullptr) {
     dim3 g(n_to / (32 * MT), n_r / 64);
-    hipLaunchKernelGGL((rad_stage_a<MO, PLAN>), dim3(n_r), dim3(LH_T), 0, s, dargs, tw, stage);
+    if (one)
+        hipLaunchKernelGGL((rad_stage_a_one<MO, PLAN>), dim3(n_r), dim3(LH_T), 0, s, one->a, one->h,
+                           const_cast<RadArgs*>(dargs), tw);
+    else
+        hipLaunchKernelGGL((rad_stage_a<MO, PLAN>), dim3(n_r), dim3(LH_T), 0, s, dargs, tw, stage);
     hipLaunchKernelGGL((rad_gemm<MT>), g, dim3(256), 0, s, dargs, 0);
     hipLaunchKernelGGL((rad_pointwise<MO>), dim3(n_r), dim3(LH_T), 0, s, dargs);
     hipLaunchKernelGGL((rad_gemm<MT>), g, dim3(256), 0, s, dargs, 1);
@@ -621,34 +659,35 @@ static bool rad_env_size_ok(int n_to) { return n_to >= 256 && n_to <= 8192 && (n
 
 // One RHS (stage < 0: of rhs_in or the current state) or one step, under plan p.
 template <int MO, int MC, int PLAN, int MT>
-static void rad_run(bool step, const RadArgs* a, const double2* tw, int n_to, int n_r, int stage, hipStream_t s) {
+static void rad_run(bool step, const RadArgs* a, const double2* tw, int n_to, int n_r, int stage, hipStream_t s,
+                    const RadOne* one) {
     if (step)
         rad_launch_step<MO, MC, PLAN, MT>(a, tw, n_to, n_r, s);
     else
-        rad_launch_rhs<MO, PLAN, MT>(a, tw, n_to, n_r, stage, s);
+        rad_launch_rhs<MO, PLAN, MT>(a, tw, n_to, n_r, stage, s, one);
 }
 
 template <int MO, int MC, int PLAN>
 static void rad_run_mt(const RadPlan& p, bool step, const RadArgs* a, const double2* tw, int n_to, int n_r, int stage,
-                       hipStream_t s) {
+                       hipStream_t s, const RadOne* one) {
     switch (rad_tiles(p, n_to, n_r)) {
-        case 1: rad_run<MO, MC, PLAN, 1>(step, a, tw, n_to, n_r, stage, s); break;
-        case 4: rad_run<MO, MC, PLAN, 4>(step, a, tw, n_to, n_r, stage, s); break;
-        default: rad_run<MO, MC, PLAN, 2>(step, a, tw, n_to, n_r, stage, s); break;
+        case 1: rad_run<MO, MC, PLAN, 1>(step, a, tw, n_to, n_r, stage, s, one); break;
+        case 4: rad_run<MO, MC, PLAN, 4>(step, a, tw, n_to, n_r, stage, s, one); break;
+        default: rad_run<MO, MC, PLAN, 2>(step, a, tw, n_to, n_r, stage, s, one); break;
     }
 }
 
 template <int MO, int MC>
 static void rad_run_plan(const RadPlan& p, bool step, const RadArgs* a, const double2* tw, int n_to, int n_r,
-                         int stage, hipStream_t s) {
+                         int stage, hipStream_t s, const RadOne* one) {
     if (p.fft == 1)
-        rad_run_mt<MO, MC, 1>(p, step, a, tw, n_to, n_r, stage, s);
+        rad_run_mt<MO, MC, 1>(p, step, a, tw, n_to, n_r, stage, s, one);
     else
-        rad_run_mt<MO, MC, 0>(p, step, a, tw, n_to, n_r, stage, s);
+        rad_run_mt<MO, MC, 0>(p, step, a, tw, n_to, n_r, stage, s, one);
 }
 
 static void rad_dispatch(const RadPlan& p, bool step, bool env, int n_to, int n_r, const RadArgs* a,
-                         const double2* tw, int stage, hipStream_t s) {
+                         const double2* tw, int stage, hipStream_t s, const RadOne* one = nullptr) {
     if (env) {  // the radix plan of the column transforms is the default one
         switch (n_to) {
             case 8192: rad_run_env_mt<8192>(p, step, a, tw, n_r, stage, s); break;
@@ -661,16 +700,16 @@ static void rad_dispatch(const RadPlan& p, bool step, bool env, int n_to, int n_
         return;
     }
     switch (n_to) {
-        case 16384: rad_run_plan<8192, 4096>(p, step, a, tw, n_to, n_r, stage, s); break;
-        case 8192: rad_run_plan<4096, 2048>(p, step, a, tw, n_to, n_r, stage, s); break;
-        case 4096: rad_run_plan<2048, 1024>(p, step, a, tw, n_to, n_r, stage, s); break;
-        default: rad_run_plan<1024, 512>(p, step, a, tw, n_to, n_r, stage, s); break;
+        case 16384: rad_run_plan<8192, 4096>(p, step, a, tw, n_to, n_r, stage, s, one); break;
+        case 8192: rad_run_plan<4096, 2048>(p, step, a, tw, n_to, n_r, stage, s, one); break;
+        case 4096: rad_run_plan<2048, 1024>(p, step, a, tw, n_to, n_r, stage, s, one); break;
+        default: rad_run_plan<1024, 512>(p, step, a, tw, n_to, n_r, stage, s, one); break;
     }
 }
 
 static void rad_rhs_dispatch(const RadPlan& p, bool env, int n_to, int n_r, const RadArgs* a, const double2* tw,
-                             int stage, hipStream_t s) {
-    rad_dispatch(p, false, env, n_to, n_r, a, tw, stage, s);
+                             int stage, hipStream_t s, const RadOne* one = nullptr) {
+    rad_dispatch(p, false, env, n_to, n_r, a, tw, stage, s, one);
 }
 
 static void rad_step_dispatch(const RadPlan& p, bool env, int n_to, int n_r, const RadArgs* a, const double2* tw,
