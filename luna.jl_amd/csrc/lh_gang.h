@@ -134,14 +134,14 @@ __device__ __forceinline__ void gang_sync(Gang& g, SM& sm) {
     g.ep++;
     const int t = threadIdx.x;
     if (t < 64) {
-        if (t == 0) lg_st(g.flags + LG_FLAG_STRIDE * g.h, (g.ep << 4) | (unsigned)(sm.flag & 15));
+        if (t == 0) lg_st(g.flags + LG_FLAG_STRIDE * g.h, lg_flag(g.ep, sm.flag));
         if (t < LG_G) {
             unsigned v = 0;
             int it = 0;
             const bool dead = sm.gflag == LH_E_HIP;
             do {
                 v = lg_ld(g.flags + LG_FLAG_STRIDE * t);
-            } while (!dead && (int)((v >> 4) - (g.ep & 0x0fffffffu)) < 0 && ++it < LG_MAX_POLL);
+            } while (!dead && lg_behind(v, g.ep) && ++it < LG_MAX_POLL);
             if (it >= LG_MAX_POLL)
                 sm.gflag = LH_E_HIP;
             else if ((v & 15u) != 0 && sm.gflag == LH_OK)

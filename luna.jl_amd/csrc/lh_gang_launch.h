@@ -5,14 +5,12 @@
 #include <string.h>
 
 #include "../../include/luna_hip.h"
+#include "lh_gang_proto.h"
 
 struct DInst;
 
-static constexpr int LG_G = 4;               // members of a gang
 static constexpr int LG_TWN = 32768;         // twiddle table: exp(-2πi m/LG_TWN)
 static constexpr int LG_MIN_WG = 32;         // workgroups of the smallest launch
-static constexpr int LG_XCC = 16;            // values of HW_REG_XCC_ID
-static constexpr int LG_FLAG_STRIDE = 32;    // unsigneds between two members' flags (one cache line)
 static constexpr int LG_SLOTS = 14;          // vectors of an instance's work block, see LgVec
 
 // Control block of one launch.
