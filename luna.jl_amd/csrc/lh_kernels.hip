@@ -567,14 +567,23 @@ static DInst base_inst(const lh_ctx* c) {
     return in;
 }
 
-// A launch over one instance: its control block and DInst, uploaded together.
+// A launch over one instance: its control block, then its DInst.  A kernel that
+// has them by value puts them there, in stream order, so no host memory has to
+// outlive the call.
 static constexpr size_t LAUNCH1_CTL = (lg_ctl_bytes(1, LG_MIN_WG) + 255) / 256 * 256;
 static constexpr size_t LAUNCH1_BYTES = LAUNCH1_CTL + (sizeof(DInst) + 255) / 256 * 256;
-static int upload_launch1(unsigned char* dst, const DInst& in, hipStream_t s) {
-    unsigned char h[LAUNCH1_CTL + sizeof(DInst)];
-    lg_ctl_init(h, 1, LG_MIN_WG);
-    memcpy(h + LAUNCH1_CTL, &in, sizeof(DInst));
-    HIPCK(hipMemcpyAsync(dst, h, sizeof(h), hipMemcpyHostToDevice, s));
+__global__ __launch_bounds__(64) void lh_set_launch1(DInst in, unsigned char* at) {
+    unsigned* ctl = (unsigned*)at;
+    for (int i = threadIdx.x; i < (int)(LAUNCH1_CTL / sizeof(unsigned)); i += 64) ctl[i] = 0u;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    ((GangCtl*)at)->njobs = 1;
+    ((GangCtl*)at)->n_wg = LG_MIN_WG;
+    *(DInst*)(at + LAUNCH1_CTL) = in;
+}
+static int set_launch1(unsigned char* at, const DInst& in, hipStream_t s) {
+    hipLaunchKernelGGL(lh_set_launch1, dim3(1), dim3(64), 0, s, in, at);
+    HIPCK(hipGetLastError());
     return LH_OK;
 }
 
@@ -1327,7 +1336,7 @@ int lh_solve_stream(lh_ctx* c, double* Ew, const lh_rk_opts* o, lh_output_cb cb,
         in.pub_info = (double*)(db + off_info);
         in.pub_y = (double2*)(db + off_y);
         in.pub_ring = every ? (int)nslot : 0;
-        st = upload_launch1(c->launch1, in, c->stream);
+        st = set_launch1(c->launch1, in, c->stream);
     }
     if (!st) {
         if (!launch_solve(launch1_of(c, c->launch1, tw, c->stream), c->d.raman != 0, true)) st = LH_E_ARG;
@@ -2118,9 +2127,9 @@ int lh_solve_noalloc(lh_ctx* c, void* Ew_dev, const lh_rk_opts* o, void* saves_d
     inst_options(&in, o);
     // Nothing in the working memory needs clearing: the kernel writes every
     // state and stage vector before reading it, and the counters at the end.
-    // Host staging lives on this stack frame; each copy is waited for before
-    // the frame's buffer is reused or left.
-    const int st = upload_launch1(base + L.inst, in, s);
+    // The save grid is staged on this stack frame; each copy is waited for
+    // before the frame's buffer is reused or left.
+    const int st = set_launch1(base + L.inst, in, s);
     if (st) return st;
     const int zn = o->save_n > 0 ? o->save_n : 1;
     double chunk[256];
