@@ -92,6 +92,7 @@ struct DInst {
     // slot k % pub_ring of pub_ring slots (pub_info and pub_y hold that many);
     // the kernel never waits, the host checks that it has not been lapped
     int pub_ring;
+    unsigned* beat;          // a word of the device that every solver changes at each step attempt
 };
 
 // Dormand–Prince tableau, src/dopri.jl:1-28 (rational literals evaluated in double).

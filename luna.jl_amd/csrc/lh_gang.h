@@ -1,6 +1,7 @@
 // lh_gang.h -- mode-averaged propagation by gangs of four workgroups (gfx950).
 //
-// Compiled by lh_gang_field.hip, lh_gang_raman.hip and lh_gang_env.hip.  One instance is
+// Compiled by lh_gang_field.hip, lh_gang_raman.hip, lh_gang_env.hip and
+// lh_gang_dense.hip.  One instance is
 // solved by a gang: four workgroups of 512 threads on four CUs of one XCD,
 // which exchange data through that XCD's L2.  A transform of M points splits
 // as M = 8·S: the bins k ≡ r (mod 8) form one S-point transform, and an
@@ -28,7 +29,9 @@
 // XCD (HW_REG_XCC_ID), and four consecutive tickets are a gang, so members are
 // resident and share an L2 whatever the order of dispatch.  Gangs then take
 // jobs (instances) from one counter until none is left.  A launch has at least
-// 32 workgroups, so that one of at most eight XCDs gets four of them.
+// 32 workgroups, so that one of at most eight XCDs gets four of them; where
+// they don't become resident there, the launch ends with LH_E_HIP
+// (lh_gang_proto.h).
 
 #pragma once
 #include "lh_core.h"
@@ -36,7 +39,8 @@
 
 typedef double lg_d2 __attribute__((ext_vector_type(2)));
 
-static constexpr int LG_MAX_POLL = 1 << 25;  // polls of a barrier before it gives up (some ten seconds)
+static constexpr int LG_MAX_POLL = 1 << 25;  // polls of another member before it counts as lost (some ten seconds)
+static_assert(LG_LOST == LH_E_HIP, "the protocol's status of a lost member");
 
 static_assert(LH_T == 512, "a gang member is 8 wavefronts, one per run of its times");
 
@@ -54,6 +58,25 @@ template <class T>
 __device__ __forceinline__ void lg_st(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// The protocol's memory operations (lh_gang_proto.h).
+struct LgMem {
+    template <class T>
+    __device__ __forceinline__ static T ld(const T* p) {
+        return lg_ld(p);
+    }
+    __device__ __forceinline__ static void st(unsigned long long* p, unsigned long long v) { lg_st(p, v); }
+    __device__ __forceinline__ static unsigned add(unsigned* p, unsigned v) {
+        return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ static unsigned long long cas(unsigned long long* p, unsigned long long old,
+                                                             unsigned long long v) {
+        __hip_atomic_compare_exchange_strong(p, &old, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return old;
+    }
+    __device__ __forceinline__ static void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+    __device__ __forceinline__ static void pause() { __builtin_amdgcn_s_sleep(8); }
+};
 
 // 16-byte loads past the CU's L1 (which may hold a line's earlier content) of
 // the series the other members wrote: a buffer descriptor over it and the
@@ -126,7 +149,8 @@ struct Gang {
 // then one lane raises the member's flag to the new epoch and four lanes poll
 // all flags.  A flag also carries the member's error status, so all members see
 // an error at the first barrier after it.  A member that another one does not
-// join within LG_MAX_POLL polls gives up with LH_E_HIP, so no wait is endless.
+// join within LG_MAX_POLL polls goes on alone with LH_E_HIP and raises its flag
+// again with that, which the late one finds there or at its next barrier.
 template <class SM>
 __device__ __forceinline__ void gang_sync(Gang& g, SM& sm) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -136,16 +160,16 @@ __device__ __forceinline__ void gang_sync(Gang& g, SM& sm) {
     if (t < 64) {
         if (t == 0) lg_st(g.flags + LG_FLAG_STRIDE * g.h, lg_flag(g.ep, sm.flag));
         if (t < LG_G) {
-            unsigned v = 0;
-            int it = 0;
-            const bool dead = sm.gflag == LH_E_HIP;
-            do {
-                v = lg_ld(g.flags + LG_FLAG_STRIDE * t);
-            } while (!dead && lg_behind(v, g.ep) && ++it < LG_MAX_POLL);
-            if (it >= LG_MAX_POLL)
-                sm.gflag = LH_E_HIP;
-            else if ((v & 15u) != 0 && sm.gflag == LH_OK)
-                sm.gflag = (int)(v & 15u);
+            // (one that goes on alone looks once)
+            const int st = lg_await<LgMem>(g.flags + LG_FLAG_STRIDE * t, g.ep, sm.gflag == LG_LOST ? 1 : LG_MAX_POLL);
+            if (__any(st != LH_OK)) {
+                if (__any(st == LG_LOST)) {
+                    sm.flag = sm.gflag = LG_LOST;
+                    if (t == 0) lg_st(g.flags + LG_FLAG_STRIDE * g.h, lg_flag(g.ep, LG_LOST));
+                } else if (st != LH_OK && sm.gflag == LH_OK) {
+                    sm.gflag = st;
+                }
+            }
         }
     }
     __syncthreads();
@@ -1220,6 +1244,7 @@ __device__ __forceinline__ void g_solve(const DInst& in, SM& sm, Gang& g) {
             h0 = tn - t;
             dt = dtn;
             t = tn;
+            if (h == 0 && threadIdx.x == 0) lg_st(in.beat, (unsigned)steps);
         }
         const int st_end = (st < 0) ? 0 : 6;
 #pragma unroll 1
@@ -1524,6 +1549,8 @@ __device__ __forceinline__ void g_solve(const DInst& in, SM& sm, Gang& g) {
         __syncthreads();
     }
     for (int p = fresh_tid(); p < nb; p += LH_T) gl(in.Y)[Z::k_of(h, p)] = gl(Y)[p];
+    gang_sync(g, sm);  // whoever lost a member says so before the record is written
+    if (sm.gflag == LG_LOST) status = LH_E_HIP;
     if (h == 0 && threadIdx.x == 0 && gl(in.stats)) {
         lh_stats s;
         s.steps = steps;
@@ -1547,55 +1574,29 @@ struct GLds {
     using T = GSmem<(KIND == 0 && RAMAN) ? M / 2 : M / 4, (KIND == 1) ? 1 : (M >= 16384 || RAMAN) ? 1024 : 2048>;
 };
 
-// Forms gangs and hands their members jobs.  run(job) is called by all members
-// of a gang together.  RESET: the control block is used by launch after launch
-// (in stream order) instead of being uploaded for each.
+// Forms gangs and hands their members jobs (lg_next_job).  run(job) is called by
+// all members of a gang together.  status: null, or where the status of a launch
+// of one job goes, whose control block then serves launch after launch (in
+// stream order) instead of being set for each.
 template <bool RESET, class SM, class F>
-__device__ __forceinline__ void gang_loop(GangCtl* ctl, SM& sm, Gang& g, F run) {
+__device__ __forceinline__ void gang_loop(GangCtl* ctl, SM& sm, Gang& g, int* status, F run) {
     const int n_gang = (int)(ctl->n_wg / LG_G);
     const unsigned njobs = ctl->njobs;
     unsigned long long* mailbox = (unsigned long long*)((char*)ctl + lg_mail_off(njobs));
     if (threadIdx.x == 0) {
         const unsigned xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20) & (LG_XCC - 1);  // HW_REG_XCC_ID, 4 bits
-        const unsigned tk = __hip_atomic_fetch_add(&ctl->ticket[xcc], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned tk = LgMem::add(&ctl->ticket[xcc], 1u);
         sm.member = (int)(tk % LG_G);
         sm.slot = (int)(xcc * n_gang + tk / LG_G);
+        sm.gflag = LH_OK;
     }
     __syncthreads();
     g.h = __builtin_amdgcn_readfirstlane(sm.member);
     unsigned long long* mail = mailbox + __builtin_amdgcn_readfirstlane(sm.slot);
-    // The last member to arrive completes the gang and leads it: it takes the
-    // jobs.  The mailbox holds (sequence << 32 | job), job 0xffffffff for "no
-    // more".  A member whose gang never completes leaves once every job has
-    // been taken: it reads the job counter first and the mailbox after it, and
-    // the leader writes "formed" (sequence 1) before it takes a job.
     unsigned seq = 1;
     for (;;) {
-        if (threadIdx.x == 0) {
-            unsigned job = 0xffffffffu;
-            if (g.h == LG_G - 1) {
-                if (seq == 1) {
-                    lg_st(mail, 1ull << 32 | 0xfffffffeull);  // formed
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                }
-                job = __hip_atomic_fetch_add(&ctl->next_job, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (job >= njobs) job = 0xffffffffu;
-                lg_st(mail, (unsigned long long)(seq + 1) << 32 | job);
-            } else {
-                for (;;) {
-                    const unsigned taken = lg_ld(&ctl->next_job);
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    const unsigned long long m = lg_ld(mail);
-                    if ((unsigned)(m >> 32) == seq + 1) {
-                        job = (unsigned)m;
-                        break;
-                    }
-                    if (m == 0 && taken >= njobs) break;  // no gang, no job
-                    __builtin_amdgcn_s_sleep(8);
-                }
-            }
-            sm.job = (int)job;
-        }
+        if (threadIdx.x == 0)
+            sm.job = (int)lg_next_job<LgMem>(ctl, mail, g.h, seq, sm.gflag == LG_LOST, njobs, LG_MAX_POLL);
         __syncthreads();
         const int job = __builtin_amdgcn_readfirstlane(sm.job);
         __syncthreads();
@@ -1607,11 +1608,15 @@ __device__ __forceinline__ void gang_loop(GangCtl* ctl, SM& sm, Gang& g, F run) 
         run(job);
     }
     if constexpr (RESET) {
-        // the last workgroup to leave makes the control block ready for the next launch
-        if (threadIdx.x == 0)
-            sm.job = (int)__hip_atomic_fetch_add(&ctl->left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the last workgroup to leave has the status of all, and makes the control
+        // block ready for the next launch
+        if (threadIdx.x == 0) {
+            const unsigned mine = lg_leave(g.h, seq - 1, sm.gflag), sum = LgMem::add(&ctl->left, mine) + mine;
+            sm.job = (sum & 255u) == ctl->n_wg;
+            if (sm.job) *status = lg_left(sum);
+        }
         __syncthreads();
-        if (sm.job == (int)ctl->n_wg - 1) {
+        if (sm.job) {
             unsigned* flags = (unsigned*)((char*)ctl + lg_flags_off());
             for (int i = threadIdx.x; i < (int)njobs * LG_G; i += LH_T) lg_st(flags + i * LG_FLAG_STRIDE, 0u);
             for (int i = threadIdx.x; i < LG_XCC * n_gang; i += LH_T) lg_st(mailbox + i, 0ull);
@@ -1643,7 +1648,7 @@ __global__ __launch_bounds__(LH_T, DENSE ? 4 : 1) void lh_gang_solve(GangCtl* ct
     __shared__ SM sm;
     gtw_load(sm.tw, twg);
     Gang g;
-    gang_loop<false>(ctl, sm, g, [&](int job) {
+    gang_loop<false>(ctl, sm, g, nullptr, [&](int job) {
         const DInst& in = insts[job];
         gang_area(g, in);
         g_solve<KIND, M, STREAM, RAMAN, DENSE>(in, sm, g);
@@ -1659,7 +1664,7 @@ __global__ __launch_bounds__(LH_T) void lh_gang_rhs(GangCtl* ctl, const DInst in
     __shared__ SM sm;
     gtw_load(sm.tw, twg);
     Gang g;
-    gang_loop<true>(ctl, sm, g, [&](int) {
+    gang_loop<true>(ctl, sm, g, status, [&](int) {
         gang_area(g, in);
         if (threadIdx.x == 0) sm.flag = sm.gflag = LH_OK;
         __syncthreads();
@@ -1687,7 +1692,6 @@ __global__ __launch_bounds__(LH_T) void lh_gang_rhs(GangCtl* ctl, const DInst in
             const int k = Z::k_of(h, p);
             gl(in.rhs_out)[k] = cmul(g_rhs_bin<KIND, M>(sm, g, p), of[zdep ? p : k]);
         }
-        if (h == 0 && threadIdx.x == 0) *status = sm.gflag;
     });
 }
 
@@ -1701,7 +1705,7 @@ __global__ __launch_bounds__(LH_T) void lh_gang_stats(GangCtl* ctl, const DInst 
     __shared__ SM sm;
     gtw_load(sm.tw, twg);
     Gang g;
-    gang_loop<true>(ctl, sm, g, [&](int) {
+    gang_loop<true>(ctl, sm, g, status, [&](int) {
         gang_area(g, in);
         if (threadIdx.x == 0) sm.flag = sm.gflag = LH_OK;
         __syncthreads();
@@ -1730,7 +1734,6 @@ __global__ __launch_bounds__(LH_T) void lh_gang_stats(GangCtl* ctl, const DInst 
             }
         }
         g_stats<KIND, M>(in, sm, g, s0, s1, se, ws, z, dz, rho, gl(in.steprec));
-        if (h == 0 && threadIdx.x == 0) *status = sm.gflag;
     });
 }
 

@@ -13,21 +13,6 @@ static constexpr int LG_TWN = 32768;         // twiddle table: exp(-2πi m/LG_TW
 static constexpr int LG_MIN_WG = 32;         // workgroups of the smallest launch
 static constexpr int LG_SLOTS = 14;          // vectors of an instance's work block, see LgVec
 
-// Control block of one launch.
-struct GangCtl {
-    unsigned next_job, njobs, n_wg, left;
-    unsigned pad[12];
-    unsigned ticket[LG_XCC];
-    // then per job LG_G flags (LG_FLAG_STRIDE apart), then mail[LG_XCC][n_wg / LG_G] (64-bit)
-};
-__host__ __device__ constexpr size_t lg_flags_off() { return sizeof(GangCtl); }
-__host__ __device__ constexpr size_t lg_mail_off(size_t njobs) {
-    return sizeof(GangCtl) + njobs * LG_G * LG_FLAG_STRIDE * sizeof(unsigned);
-}
-__host__ __device__ constexpr size_t lg_ctl_bytes(size_t njobs, size_t n_wg) {
-    return lg_mail_off(njobs) + LG_XCC * (n_wg / LG_G) * sizeof(unsigned long long);
-}
-
 // Complex points of a transform and the work block of a mode-averaged class.
 static inline int lg_points(const lh_desc& d) { return d.grid_kind == LH_GRID_REAL ? d.n_to / 2 : d.n_to; }
 static inline size_t lg_stride(const lh_desc& d) {  // one vector of the work block
@@ -58,11 +43,12 @@ static inline int lg_workgroups(int n, double share, bool dense) {
 // workgroup per CU / two: 128 23.2/29.0, 160 27.7/29.7, 192 34.4/30.3, 224
 // 38.8/33.2, 256 44.6/40.0; 384 of 0.2 m 35.3/34.0.
 static constexpr int LG_DENSE_ABOVE = 176;
-static inline void lg_ctl_init(void* p, int njobs, int nwg) {
+static inline void lg_ctl_init(void* p, int njobs, int nwg, const unsigned* beat) {
     memset(p, 0, lg_ctl_bytes(njobs, nwg));
     GangCtl* c = (GangCtl*)p;
     c->njobs = (unsigned)njobs;
     c->n_wg = (unsigned)nwg;
+    c->beat = beat;
 }
 
 // Launches of a class over the instances d (job i is d[i]; device memory for a

@@ -225,6 +225,7 @@ struct lh_ctx {
     int zgrid_hn;
     lh_stats* dstats;
     unsigned char* launch1;  // one instance's solve: control block, then its DInst
+    unsigned* beat;          // the device's
     GangCtl* rhs_ctl;        // control block of single right-hand sides and records (reset by each launch)
     hipEvent_t rhs_ev;       // orders those launches when they change streams
     double2* rhs_in;
@@ -282,6 +283,9 @@ static double2* g_gtw[64] = {nullptr};
 static constexpr size_t SCRATCH_BYTES = LH_NOALLOC_SCRATCH_BYTES + (1024u * 1024u);
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 static unsigned char* g_scratch[64] = {nullptr};
+// The word of each GPU that its solvers change as they get on (GangCtl::beat).
+static __device__ unsigned beat;
+static unsigned* g_beat[64] = {nullptr};
 // HIP-event durations of the last resident batch, per size class
 static float g_last_ms[8] = {0};
 static int g_last_n[8] = {0};
@@ -327,14 +331,17 @@ static void sincos_frac(long m, long N, double* c, double* s) {
     *s = (double)S;
 }
 
-// Device address of `scratch` on dev (the current device), looked up once.
+// Device addresses of `scratch` and `beat` on dev (the current device), looked up once.
 static int scratch_init(int dev) {
     std::lock_guard<std::mutex> g(g_mu);
     if (dev < 0 || dev >= 64) return LH_E_ARG;
     if (!g_scratch[dev]) {
         void* p = nullptr;
         HIPCK(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-        if (!p) return LH_E_HIP;
+        void* b = nullptr;
+        HIPCK(hipGetSymbolAddress(&b, HIP_SYMBOL(beat)));
+        if (!p || !b) return LH_E_HIP;
+        g_beat[dev] = (unsigned*)b;
         g_scratch[dev] = (unsigned char*)p;
     }
     return LH_OK;
@@ -506,6 +513,7 @@ static DInst base_inst(const lh_ctx* c) {
     in.escr = c->escr;
     in.gx = c->gx;
     in.gx_len = (int)lg_exchange_len(d);
+    in.beat = c->beat;
     in.ionpot = d.ionpot;
     in.preion_p1 = d.preionfrac + 1;
     in.e_ratio = ECHARGE * ECHARGE / MELEC;
@@ -567,6 +575,12 @@ static DInst base_inst(const lh_ctx* c) {
     return in;
 }
 
+// The counters of an instance until its solver writes them: what a launch whose
+// gangs never form leaves.
+__host__ __device__ static lh_stats unsolved(const DInst& in) {
+    return lh_stats{0, 0, 0, 0, LH_E_HIP, in.save_first, in.z0, in.init_dz};
+}
+
 // A launch over one instance: its control block, then its DInst.  A kernel that
 // has them by value puts them there, in stream order, so no host memory has to
 // outlive the call.
@@ -579,7 +593,9 @@ __global__ __launch_bounds__(64) void lh_set_launch1(DInst in, unsigned char* at
     if (threadIdx.x != 0) return;
     ((GangCtl*)at)->njobs = 1;
     ((GangCtl*)at)->n_wg = LG_MIN_WG;
+    ((GangCtl*)at)->beat = in.beat;
     *(DInst*)(at + LAUNCH1_CTL) = in;
+    *in.stats = unsolved(in);
 }
 static int set_launch1(unsigned char* at, const DInst& in, hipStream_t s) {
     hipLaunchKernelGGL(lh_set_launch1, dim3(1), dim3(64), 0, s, in, at);
@@ -1084,6 +1100,7 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
     int st = LH_OK;
     if (hipGetDevice(&c->device) != hipSuccess) st = LH_E_HIP;
     if (!st) st = scratch_init(c->device);
+    if (!st) c->beat = g_beat[c->device];
     if (!st && hipStreamCreate(&c->stream) != hipSuccess) st = LH_E_HIP;
     const size_t N = (size_t)d->n_omega, NS = (size_t)c->n_state;
     if (!st) st = shared_upload(c->device, &c->omega_win, d->omega_win, N);
@@ -1155,7 +1172,7 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
     if (!st && modeavg && hipMalloc(&c->launch1, LAUNCH1_BYTES + LAUNCH1_CTL) != hipSuccess) st = LH_E_NOMEM;
     if (!st && modeavg) {
         unsigned char h[LAUNCH1_CTL];
-        lg_ctl_init(h, 1, LG_MIN_WG);
+        lg_ctl_init(h, 1, LG_MIN_WG, c->beat);
         c->rhs_ctl = (GangCtl*)(c->launch1 + LAUNCH1_BYTES);
         if (hipMemcpy(c->rhs_ctl, h, sizeof(h), hipMemcpyHostToDevice) != hipSuccess) st = LH_E_HIP;
     }
@@ -1592,17 +1609,18 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         if (count[c] && c < V_ZDEP * LH_NCLASS && c != LH_CLASS_RADIAL)
             total += up(lg_ctl_bytes(count[c], nwg[c]));
     }
-    const size_t in_bytes = total;
+    const size_t st_off = total, in_bytes = st_off + sizeof(lh_stats) * (size_t)n;
     unsigned char* dblk = nullptr;
-    HIPCK(hipMalloc(&dblk, in_bytes + sizeof(lh_stats) * (size_t)n));
+    HIPCK(hipMalloc(&dblk, in_bytes));
     const DInst* dinst = (const DInst*)dblk;
-    lh_stats* dstats = (lh_stats*)(dblk + in_bytes);
+    lh_stats* dstats = (lh_stats*)(dblk + st_off);
     std::vector<unsigned char> hblk(in_bytes);
     DInst* h = (DInst*)hblk.data();
     for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
-        if (count[c] && c != LH_CLASS_RADIAL) lg_ctl_init(hblk.data() + ctl_off[c], count[c], nwg[c]);
+        if (count[c] && c != LH_CLASS_RADIAL) lg_ctl_init(hblk.data() + ctl_off[c], count[c], nwg[c], ctxs[0]->beat);
     for (int i = 0; i < n && !st; i++)
         st = prepare_instance(ctxs[i], op[i], want_saves != 0, &h[pos[i]], dstats + pos[i], s0);
+    for (int i = 0; i < n && !st; i++) ((lh_stats*)(hblk.data() + st_off))[i] = unsolved(h[i]);
     if (!st && hipMemcpyAsync(dblk, hblk.data(), in_bytes, hipMemcpyHostToDevice, s0) != hipSuccess) st = LH_E_HIP;
     std::vector<lh_stats> rad_stats(n);
     hipEvent_t ready = nullptr, done[NG] = {nullptr}, t0[NG] = {nullptr}, t1[NG] = {nullptr};

@@ -776,6 +776,8 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
         double h0 = tn - t;
         dt = dtn;
         t = tn;
+        if (threadIdx.x == 0)
+            __hip_atomic_store(in.beat, (unsigned)steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // prop!(ks[1], t, tn) with the operator at tn; each stage then
         // re-evaluates it at its own t2
         if constexpr (ZDEP) {
