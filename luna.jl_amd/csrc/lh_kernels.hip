@@ -205,7 +205,7 @@ struct lh_ctx {
     double2* outfac;
     double4* ppt;
     double2* hwdt;  // envelope Raman: rfft(h, 2·Nto)·δt
-    double2* escr;  // field-grid Raman: E(t) and P(t), Nto/2 points each
+    double2* escr;  // field-grid Raman: E(t) and P(t), Nto/2 points each: solves, then right-hand sides
     double2* gx;    // exchange areas of the gang: solves, then single right-hand sides and records
     // solver buffers (allocated on first use)
     double2* Yin;
@@ -263,7 +263,7 @@ struct lh_ctx {
     double4* zd;                       // shared
     double2 *znwg, *zpre;              // shared
     unsigned char* zsidx;              // shared
-    double2 *zL, *zOF;                 // per context
+    double2 *zL, *zOF;                 // per context: solves, then right-hand sides
     int zg_taper;                      // 1 linear, 2 piecewise-linear taper
     double zg_a0, zg_a1, zg_aL, zg_sqrt_intg;
     int zt_n;
@@ -605,6 +605,20 @@ static int set_launch1(unsigned char* at, const DInst& in, hipStream_t s) {
 
 static GangLaunch launch1_of(const lh_ctx* c, unsigned char* at, const double2* tw, hipStream_t s) {
     return {ctx_class(c), LG_MIN_WG, (GangCtl*)at, (const DInst*)(at + LAUNCH1_CTL), tw, s};
+}
+
+// The record of a single right-hand side or statistics record: an exchange area,
+// Raman series, operator and output factor other than the solver's, so that an
+// asynchronous call and a solve of one context may overlap.
+static DInst rhs_inst(const lh_ctx* c) {
+    DInst in = base_inst(c);
+    in.gx += lg_area_len(c->d);
+    if (in.escr) in.escr += c->d.n_to;
+    if (c->zg_on) {
+        in.zL += lg_stride(c->d);
+        in.zOF += lg_stride(c->d);
+    }
+    return in;
 }
 
 // A single right-hand side or record on stream s: the context's launches share
@@ -1142,7 +1156,7 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
     const bool modeavg = d->transform == LH_TRANS_MODEAVG;
     const bool field_raman = modeavg && d->grid_kind == LH_GRID_REAL && d->raman;
     if (!st && ctx_class(c) == LH_CLASS_32768 && d->raman) st = LH_E_ARG;  // no Raman convolution on the largest field grid
-    if (!st && field_raman && hipMalloc(&c->escr, sizeof(double2) * (size_t)d->n_to) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && field_raman && hipMalloc(&c->escr, sizeof(double2) * 2 * (size_t)d->n_to) != hipSuccess) st = LH_E_NOMEM;
     if (!st && modeavg && hipMalloc(&c->gx, sizeof(double2) * 2 * lg_area_len(*d)) != hipSuccess) st = LH_E_NOMEM;
     if (!st && d->raman) {
         const double2* tw;
@@ -1219,11 +1233,10 @@ int lh_rhs_device(lh_ctx* c, void* nl_dev, const void* Ew_dev, double z, void* s
         if (env) hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, one.a, one.h, c->rargs + 1);
         rad_rhs_dispatch(c->rplan, env, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s, &one);
     } else {
-        DInst in = base_inst(c);
+        DInst in = rhs_inst(c);
         in.rhs_in = (const double2*)Ew_dev;
         in.rhs_out = (double2*)nl_dev;
         in.z0 = z;  // a gradient fill evaluates its constants at z
-        in.gx += lg_area_len(c->d);
         GangLaunch l;
         st = rhs_launch_of(c, &in, tw, s, &l);
         if (st) return st;
@@ -1828,8 +1841,8 @@ int lh_set_gradient(lh_ctx* c, const lh_gradient_desc* g) {
     if (!st && g->taper) st = shared_upload(c->device, &c->zfdt, g->fdt, (size_t)27);
     if (!st && g->taper == 2) st = shared_upload(c->device, &c->zt_Z, g->taper_Z, (size_t)g->taper_n);
     if (!st && g->taper == 2) st = shared_upload(c->device, &c->zt_A, g->taper_A, (size_t)g->taper_n);
-    if (!st && !c->zL && hipMalloc(&c->zL, sizeof(double2) * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && !c->zOF && hipMalloc(&c->zOF, sizeof(double2) * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && !c->zL && hipMalloc(&c->zL, sizeof(double2) * 2 * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && !c->zOF && hipMalloc(&c->zOF, sizeof(double2) * 2 * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
     if (st) {
         zg_release(c);
         c->zg_on = 0;
@@ -1863,11 +1876,10 @@ int lh_stats_eval(lh_ctx* c, const double* Ew, double z, double dz, double* rec)
     const double2* tw;
     int st = gang_twiddles(c->device, &tw);
     if (st) return st;
-    DInst in = base_inst(c);
+    DInst in = rhs_inst(c);
     in.rhs_in = c->rhs_in;
     in.steprec = c->st_rec1;
     HIPCK(hipMemcpyAsync(c->rhs_in, Ew, bytes, hipMemcpyHostToDevice, c->stream));
-    in.gx += lg_area_len(c->d);
     GangLaunch l;
     st = rhs_launch_of(c, &in, tw, c->stream, &l);
     if (st) return st;

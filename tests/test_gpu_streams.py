@@ -1,4 +1,5 @@
-"""Calls on the caller's streams: a solve without allocations behind other work."""
+"""Calls on the caller's streams: a solve without allocations behind other work,
+right-hand sides that overlap a solve of the same context."""
 import ctypes as C
 
 import numpy as np
@@ -87,3 +88,25 @@ def test_noalloc_behind_other_work(hip, capi):
     rc = capi.lib().lh_solve_noalloc(ctx.handle, state, C.byref(opts), saves, None, C.byref(st2), s)
     assert rc == 0 and (st2.steps, st2.rejected, st2.saved) == (st.steps, st.rejected, st.saved)
     assert np.array_equal(hip.get(state, E), E) and np.array_equal(hip.get(saves, sv), sv)
+
+
+@pytest.mark.parametrize("gas,pressure,n_to", [("N2", 0.5, 8192), ("He", (0.5, 1.0), 8192), ("He", 1.0, 4096)])
+def test_rhs_beside_a_solve(hip, capi, gas, pressure, n_to):
+    """Asynchronous right-hand sides (Raman gas, gradient fill at another z,
+    constant fill) and a solve of the same context at the same time."""
+    print(f"case: rhs beside a solve, {gas} {pressure}", flush=True)
+    from luna_jl_amd import runtime
+    holder, E0 = field(n_to, gas, pressure)
+    ctx = runtime.Context(holder)
+    opts = capi.rk_opts(0.01, save_n=3, init_dz=1e-3)
+    E, sv, _, st = ctx.solve(E0, opts)
+    nl = ctx.rhs(E0, 0.04)
+    inp, out, s = hip.put(E0), hip.put(np.zeros_like(E0)), hip.stream()
+    for _ in range(3):
+        for _ in range(300):
+            rhs(capi, ctx, out, inp, s, 0.04)
+        E2, sv2, _, st2 = ctx.solve(E0, opts)
+        assert st2.steps == st.steps and np.array_equal(E2, E) and np.array_equal(sv2, sv)
+        hip.sync(s)
+        assert capi.lib().lh_ctx_status(ctx.handle) == 0
+        assert np.array_equal(hip.get(out, nl), nl)
