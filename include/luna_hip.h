@@ -158,8 +158,13 @@ int lh_destroy(lh_ctx *ctx);
  * nl, Ew: complex [n_omega*n_r].  Synchronous. */
 int lh_rhs(lh_ctx *ctx, double *nl, const double *Ew, double z);
 
-/* Same on device pointers, enqueued on stream (hipStream_t, NULL = default).
- * Errors from inside the kernel are reported by lh_ctx_status after a sync. */
+/* Same on device pointers, enqueued on stream (hipStream_t, NULL = the
+ * context's own).  Errors from inside the kernel are reported by lh_ctx_status
+ * after a sync.  On a mode-averaged context, calls on different streams may
+ * overlap with each other and with a solve; they can be captured into a graph
+ * (the captured calls of one context share working memory, so graphs that hold
+ * some are replayed one after another).  A radial context's calls share
+ * working memory with each other and with its solves: order them. */
 int lh_rhs_device(lh_ctx *ctx, void *nl_dev, const void *Ew_dev, double z, void *stream);
 int lh_ctx_status(lh_ctx *ctx);
 

@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <math.h>
+#include <pthread.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -192,6 +193,23 @@ static const double ECHARGE = 1.6021766208e-19;
 static const double MELEC = 9.10938356e-31;
 static const double CLIGHT = 299792458.0;
 
+// What the single right-hand sides and statistics records launched on one
+// stream use: a control block (which each launch leaves ready for the next), a
+// status word, an exchange area and, on a field grid with Raman, its series; in
+// z, the operator and output factor of a z-dependent fill.  A set belongs to
+// one stream, so launches on different streams share nothing, and launches on
+// one follow each other.  Launches under capture have one of their own: which
+// streams replay a graph, and beside what, is not known when it is recorded.
+// That set and one more are there from the start.
+struct RhsSet {
+    hipStream_t s;
+    unsigned long long thread;  // of hipStreamPerThread, one handle for every thread's stream
+    unsigned long long used;    // of the context's launches, the last here
+    unsigned char* block;
+    double2* z;
+};
+enum { RHS_CAPTURED, RHS_FIRST, RHS_SETS = RHS_FIRST + 5 };
+
 struct lh_ctx {
     int device;
     hipStream_t stream;
@@ -205,8 +223,8 @@ struct lh_ctx {
     double2* outfac;
     double4* ppt;
     double2* hwdt;  // envelope Raman: rfft(h, 2·Nto)·δt
-    double2* escr;  // field-grid Raman: E(t) and P(t), Nto/2 points each: solves, then right-hand sides
-    double2* gx;    // exchange areas of the gang: solves, then single right-hand sides and records
+    double2* escr;  // field-grid Raman: E(t) and P(t), Nto/2 points each, of solves
+    double2* gx;    // exchange area of the gang, of solves
     // solver buffers (allocated on first use)
     double2* Yin;
     int have_state;
@@ -226,11 +244,14 @@ struct lh_ctx {
     lh_stats* dstats;
     unsigned char* launch1;  // one instance's solve: control block, then its DInst
     unsigned* beat;          // the device's
-    GangCtl* rhs_ctl;        // control block of single right-hand sides and records (reset by each launch)
-    hipEvent_t rhs_ev;       // orders those launches when they change streams
+    RhsSet rset[RHS_SETS];
+    unsigned long long rhs_calls;
+    hipStream_t cap_stream;      // of the last launch under capture, and its capture
+    unsigned long long cap_id;
+    hipEvent_t cap_ev;
     double2* rhs_in;
     double2* rhs_out;
-    int* dstatus;
+    int* dstatus;                // of the last right-hand side or record (mode-averaged: its set's)
     int last_status;
     int rhs_pending;
     hipStream_t rhs_stream;
@@ -263,7 +284,7 @@ struct lh_ctx {
     double4* zd;                       // shared
     double2 *znwg, *zpre;              // shared
     unsigned char* zsidx;              // shared
-    double2 *zL, *zOF;                 // per context: solves, then right-hand sides
+    double2 *zL, *zOF;                 // per context, of solves
     int zg_taper;                      // 1 linear, 2 piecewise-linear taper
     double zg_a0, zg_a1, zg_aL, zg_sqrt_intg;
     int zt_n;
@@ -586,14 +607,17 @@ __host__ __device__ static lh_stats unsolved(const DInst& in) {
 // outlive the call.
 static constexpr size_t LAUNCH1_CTL = (lg_ctl_bytes(1, LG_MIN_WG) + 255) / 256 * 256;
 static constexpr size_t LAUNCH1_BYTES = LAUNCH1_CTL + (sizeof(DInst) + 255) / 256 * 256;
-__global__ __launch_bounds__(64) void lh_set_launch1(DInst in, unsigned char* at) {
-    unsigned* ctl = (unsigned*)at;
-    for (int i = threadIdx.x; i < (int)(LAUNCH1_CTL / sizeof(unsigned)); i += 64) ctl[i] = 0u;
+__device__ __forceinline__ void lg_ctl_clear(unsigned* ctl, size_t bytes, const unsigned* beat) {
+    for (int i = threadIdx.x; i < (int)(bytes / sizeof(unsigned)); i += 64) ctl[i] = 0u;
     __syncthreads();
     if (threadIdx.x != 0) return;
-    ((GangCtl*)at)->njobs = 1;
-    ((GangCtl*)at)->n_wg = LG_MIN_WG;
-    ((GangCtl*)at)->beat = in.beat;
+    ((GangCtl*)ctl)->njobs = 1;
+    ((GangCtl*)ctl)->n_wg = LG_MIN_WG;
+    ((GangCtl*)ctl)->beat = beat;
+}
+__global__ __launch_bounds__(64) void lh_set_launch1(DInst in, unsigned char* at) {
+    lg_ctl_clear((unsigned*)at, LAUNCH1_CTL, in.beat);
+    if (threadIdx.x != 0) return;
     *(DInst*)(at + LAUNCH1_CTL) = in;
     *in.stats = unsolved(in);
 }
@@ -607,40 +631,74 @@ static GangLaunch launch1_of(const lh_ctx* c, unsigned char* at, const double2* 
     return {ctx_class(c), LG_MIN_WG, (GangCtl*)at, (const DInst*)(at + LAUNCH1_CTL), tw, s};
 }
 
-// The record of a single right-hand side or statistics record: an exchange area,
-// Raman series, operator and output factor other than the solver's, so that an
-// asynchronous call and a solve of one context may overlap.
-static DInst rhs_inst(const lh_ctx* c) {
-    DInst in = base_inst(c);
-    in.gx += lg_area_len(c->d);
-    if (in.escr) in.escr += c->d.n_to;
-    if (c->zg_on) {
-        in.zL += lg_stride(c->d);
-        in.zOF += lg_stride(c->d);
+static bool field_raman(const lh_desc& d) {
+    return d.transform == LH_TRANS_MODEAVG && d.grid_kind == LH_GRID_REAL && d.raman;
+}
+static constexpr size_t RHS_STATUS = LAUNCH1_CTL, RHS_GX = LAUNCH1_CTL + 256;
+__global__ __launch_bounds__(64) void lh_clear_ctl(unsigned* ctl, const unsigned* beat) {
+    lg_ctl_clear(ctl, LAUNCH1_CTL, beat);
+}
+// Makes a set ready for launches on s (ordered on s; allocates what is missing).
+static int rhs_set_ready(lh_ctx* c, RhsSet* r, hipStream_t s) {
+    if (!r->block) {
+        HIPCK(hipMalloc(&r->block, RHS_GX + sizeof(double2) * (lg_area_len(c->d) + (field_raman(c->d) ? (size_t)c->d.n_to : 0))));
+        hipLaunchKernelGGL(lh_clear_ctl, dim3(1), dim3(64), 0, s, (unsigned*)r->block, c->beat);
+        HIPCK(hipGetLastError());
     }
-    return in;
+    if (c->zg_on && !r->z) HIPCK(hipMalloc(&r->z, sizeof(double2) * 2 * lg_stride(c->d)));
+    return LH_OK;
 }
 
-// A single right-hand side or record on stream s: the context's launches share
-// its control block and exchange area, so one on another stream than the last
-// waits for that one.
-static int rhs_launch_of(lh_ctx* c, const DInst* in, const double2* tw, hipStream_t s, GangLaunch* l) {
-    // a stream under capture neither waits for work outside its graph nor is
-    // waited for: the caller orders a graph's replays with its other calls
-    const auto capturing = [](hipStream_t q) {
+// The set of a launch on s.  A capture that forks runs its branches side by
+// side: a launch on another of its streams than the last one follows that one
+// inside the graph.
+static int rhs_set_of(lh_ctx* c, hipStream_t s, RhsSet** out) {
+    if (s != c->stream) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(q, &cs) != hipSuccess) (void)hipGetLastError();
-        return cs != hipStreamCaptureStatusNone;
-    };
-    if (c->rhs_stream && c->rhs_stream != s && !capturing(s) && !capturing(c->rhs_stream)) {
-        if (!c->rhs_ev) HIPCK(hipEventCreateWithFlags(&c->rhs_ev, hipEventDisableTiming));
-        if (hipEventRecord(c->rhs_ev, c->rhs_stream) != hipSuccess || hipStreamWaitEvent(s, c->rhs_ev, 0) != hipSuccess) {
-            (void)hipGetLastError();  // the caller has destroyed that stream
-            HIPCK(hipDeviceSynchronize());
+        unsigned long long id = 0;
+        HIPCK(hipStreamGetCaptureInfo(s, &cs, &id));
+        if (cs != hipStreamCaptureStatusNone) {
+            if (c->cap_stream && c->cap_id == id && c->cap_stream != s) {
+                HIPCK(hipEventRecord(c->cap_ev, c->cap_stream));
+                HIPCK(hipStreamWaitEvent(s, c->cap_ev, 0));
+            }
+            c->cap_stream = s;
+            c->cap_id = id;
+            *out = &c->rset[RHS_CAPTURED];
+            return LH_OK;  // ready since lh_create or lh_set_gradient
         }
     }
-    c->rhs_stream = s;
-    *l = {ctx_class(c), LG_MIN_WG, c->rhs_ctl, in, tw, s};
+    const unsigned long long thread = s == hipStreamPerThread ? (unsigned long long)pthread_self() : 0;
+    RhsSet* r = nullptr;
+    for (int i = RHS_FIRST; i < RHS_SETS && !r; i++)
+        if (c->rset[i].used && c->rset[i].s == s && c->rset[i].thread == thread) r = &c->rset[i];
+    if (!r) {  // a stream not seen yet: an unused set, or the one unused for longest once its launches are done
+        r = &c->rset[RHS_FIRST];
+        for (int i = RHS_FIRST + 1; i < RHS_SETS; i++)
+            if (c->rset[i].used < r->used) r = &c->rset[i];
+        if (r->used) HIPCK(hipDeviceSynchronize());
+        r->s = s;
+        r->thread = thread;
+    }
+    r->used = ++c->rhs_calls;
+    *out = r;
+    return rhs_set_ready(c, r, s);
+}
+
+// A single right-hand side or record on stream s: *in gets the memory of the
+// stream's set.
+static int rhs_launch_of(lh_ctx* c, DInst* in, const double2* tw, hipStream_t s, GangLaunch* l) {
+    RhsSet* r;
+    const int st = rhs_set_of(c, s, &r);
+    if (st) return st;
+    in->gx = (double2*)(r->block + RHS_GX);
+    if (in->escr) in->escr = in->gx + lg_area_len(c->d);
+    if (c->zg_on) {
+        in->zL = r->z;
+        in->zOF = r->z + lg_stride(c->d);
+    }
+    c->dstatus = (int*)(r->block + RHS_STATUS);
+    *l = {ctx_class(c), LG_MIN_WG, (GangCtl*)r->block, in, tw, s};
     return LH_OK;
 }
 
@@ -1083,7 +1141,7 @@ int lh_destroy(lh_ctx* c) {
                           (const void*)c->znwg, (const void*)c->zpre, (const void*)c->zsidx})
         shared_release(p);
     void* ptrs[] = {c->linop, c->outfac, c->hwdt, c->escr, c->gx, c->Yin, c->Y, c->YN,
-                    c->saves, c->zgrid, c->dstats, c->launch1, c->rhs_in, c->rhs_out, c->dstatus,
+                    c->saves, c->zgrid, c->dstats, c->launch1, c->rhs_in, c->rhs_out,
                     c->steprec, c->st_rec1, c->zL, c->zOF};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -1092,7 +1150,11 @@ int lh_destroy(lh_ctx* c) {
     for (void* p : rptrs)
         if (p) hipFree(p);
     if (c->rgraph) hipGraphExecDestroy(c->rgraph);
-    if (c->rhs_ev) hipEventDestroy(c->rhs_ev);
+    for (RhsSet& r : c->rset) {
+        if (r.block) hipFree(r.block);
+        if (r.z) hipFree(r.z);
+    }
+    if (c->cap_ev) hipEventDestroy(c->cap_ev);
     free(c->zgrid_h);
     if (c->stream) hipStreamDestroy(c->stream);
     free(c);
@@ -1154,10 +1216,9 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
         st = shared_upload(c->device, &c->ppt, p.data(), p.size());
     }
     const bool modeavg = d->transform == LH_TRANS_MODEAVG;
-    const bool field_raman = modeavg && d->grid_kind == LH_GRID_REAL && d->raman;
     if (!st && ctx_class(c) == LH_CLASS_32768 && d->raman) st = LH_E_ARG;  // no Raman convolution on the largest field grid
-    if (!st && field_raman && hipMalloc(&c->escr, sizeof(double2) * 2 * (size_t)d->n_to) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && modeavg && hipMalloc(&c->gx, sizeof(double2) * 2 * lg_area_len(*d)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && field_raman(*d) && hipMalloc(&c->escr, sizeof(double2) * (size_t)d->n_to) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && modeavg && hipMalloc(&c->gx, sizeof(double2) * lg_area_len(*d)) != hipSuccess) st = LH_E_NOMEM;
     if (!st && d->raman) {
         const double2* tw;
         double* dh = nullptr;
@@ -1183,15 +1244,13 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
         const double2* tw;
         st = modeavg ? gang_twiddles(c->device, &tw) : twiddles(c->device, &tw);
     }
-    if (!st && modeavg && hipMalloc(&c->launch1, LAUNCH1_BYTES + LAUNCH1_CTL) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && modeavg) {
-        unsigned char h[LAUNCH1_CTL];
-        lg_ctl_init(h, 1, LG_MIN_WG, c->beat);
-        c->rhs_ctl = (GangCtl*)(c->launch1 + LAUNCH1_BYTES);
-        if (hipMemcpy(c->rhs_ctl, h, sizeof(h), hipMemcpyHostToDevice) != hipSuccess) st = LH_E_HIP;
-    }
+    if (!st && modeavg && hipMalloc(&c->launch1, LAUNCH1_BYTES) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && modeavg) st = rhs_set_ready(c, &c->rset[RHS_FIRST], c->stream);
+    if (!st && modeavg) st = rhs_set_ready(c, &c->rset[RHS_CAPTURED], c->stream);
+    if (!st && modeavg &&
+        (hipEventCreateWithFlags(&c->cap_ev, hipEventDisableTiming) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess))
+        st = LH_E_HIP;
     if (!st && hipMalloc(&c->dstats, sizeof(lh_stats)) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && hipMalloc(&c->dstatus, sizeof(int)) != hipSuccess) st = LH_E_NOMEM;
     if (st) {
         lh_destroy(c);
         return st;
@@ -1233,7 +1292,7 @@ int lh_rhs_device(lh_ctx* c, void* nl_dev, const void* Ew_dev, double z, void* s
         if (env) hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, one.a, one.h, c->rargs + 1);
         rad_rhs_dispatch(c->rplan, env, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s, &one);
     } else {
-        DInst in = rhs_inst(c);
+        DInst in = base_inst(c);
         in.rhs_in = (const double2*)Ew_dev;
         in.rhs_out = (double2*)nl_dev;
         in.z0 = z;  // a gradient fill evaluates its constants at z
@@ -1841,8 +1900,8 @@ int lh_set_gradient(lh_ctx* c, const lh_gradient_desc* g) {
     if (!st && g->taper) st = shared_upload(c->device, &c->zfdt, g->fdt, (size_t)27);
     if (!st && g->taper == 2) st = shared_upload(c->device, &c->zt_Z, g->taper_Z, (size_t)g->taper_n);
     if (!st && g->taper == 2) st = shared_upload(c->device, &c->zt_A, g->taper_A, (size_t)g->taper_n);
-    if (!st && !c->zL && hipMalloc(&c->zL, sizeof(double2) * 2 * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && !c->zOF && hipMalloc(&c->zOF, sizeof(double2) * 2 * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && !c->zL && hipMalloc(&c->zL, sizeof(double2) * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && !c->zOF && hipMalloc(&c->zOF, sizeof(double2) * lg_stride(d)) != hipSuccess) st = LH_E_NOMEM;
     if (st) {
         zg_release(c);
         c->zg_on = 0;
@@ -1862,7 +1921,12 @@ int lh_set_gradient(lh_ctx* c, const lh_gradient_desc* g) {
     c->zg_sqrt_intg = g->sqrt_aeff_intg;
     c->zt_n = (g->taper == 2) ? g->taper_n : 0;
     c->zg_on = 1;
-    return LH_OK;
+    st = rhs_set_ready(c, &c->rset[RHS_CAPTURED], c->stream);
+    if (st) {
+        zg_release(c);
+        c->zg_on = 0;
+    }
+    return st;
 }
 
 int lh_stats_eval(lh_ctx* c, const double* Ew, double z, double dz, double* rec) {
@@ -1876,7 +1940,7 @@ int lh_stats_eval(lh_ctx* c, const double* Ew, double z, double dz, double* rec)
     const double2* tw;
     int st = gang_twiddles(c->device, &tw);
     if (st) return st;
-    DInst in = rhs_inst(c);
+    DInst in = base_inst(c);
     in.rhs_in = c->rhs_in;
     in.steprec = c->st_rec1;
     HIPCK(hipMemcpyAsync(c->rhs_in, Ew, bytes, hipMemcpyHostToDevice, c->stream));
