@@ -408,7 +408,11 @@ int lh_host_free(void *ptr);
  * mode-averaged grids run one persistent kernel per size class with a fixed
  * radix plan.
  *   lh_get_plan / lh_set_plan  the context's plan (a set drops the captured
- *                              step graph, re-captured on the next solve)
+ *                              step graph, re-captured on the next solve).
+ *                              Without wisdom or a set it is the default plan
+ *                              (0, 2), run with one tile on small grids
+ *   lh_plan_tiles  the tiles that the context's launches run with: the plan's,
+ *                 except for the default plan on a small grid
  *   lh_autotune   times every plan on one RHS of the field Ew (host, complex
  *                 [n_omega·n_r]; NULL: a zero field), reps timed launches
  *                 each after one untimed; installs the fastest plan whose RHS
@@ -431,6 +435,7 @@ typedef struct lh_plan {
 } lh_plan;
 int lh_get_plan(const lh_ctx *ctx, lh_plan *plan);
 int lh_set_plan(lh_ctx *ctx, const lh_plan *plan);
+int lh_plan_tiles(const lh_ctx *ctx, int *tiles);
 int lh_autotune(lh_ctx *ctx, const double *Ew, int reps, lh_plan *tried, int cap, int *n_tried);
 int lh_wisdom_export(char *buf, size_t cap, size_t *len);
 int lh_wisdom_import(const char *text);

@@ -214,6 +214,7 @@ def lib():
                                    C.POINTER(LhStats), C.c_void_p]
     L.lh_get_plan.argtypes = [C.c_void_p, C.POINTER(LhPlan)]
     L.lh_set_plan.argtypes = [C.c_void_p, C.POINTER(LhPlan)]
+    L.lh_plan_tiles.argtypes = [C.c_void_p, C.POINTER(C.c_int)]
     L.lh_autotune.argtypes = [C.c_void_p, _dp, C.c_int, C.POINTER(LhPlan), C.c_int, C.POINTER(C.c_int)]
     L.lh_wisdom_export.argtypes = [C.c_char_p, C.c_size_t, C.POINTER(C.c_size_t)]
     L.lh_wisdom_import.argtypes = [C.c_char_p]
@@ -241,7 +242,7 @@ EXPORTED = ["lh_strerror", "lh_device_count", "lh_create", "lh_destroy", "lh_rhs
             "lh_rhs_device", "lh_ctx_status", "lh_solve", "lh_solve_stream", "lh_batch_solve", "lh_batch_solve_opts", "lh_set_state",
             "lh_batch_solve_resident", "lh_get_state", "lh_get_saves", "lh_last_launch_times",
             "lh_host_alloc", "lh_host_free", "lh_solve_noalloc",
-            "lh_get_plan", "lh_set_plan", "lh_autotune", "lh_wisdom_export", "lh_wisdom_import", "lh_wisdom_forget",
+            "lh_get_plan", "lh_set_plan", "lh_plan_tiles", "lh_autotune", "lh_wisdom_export", "lh_wisdom_import", "lh_wisdom_forget",
             "lh_set_step_stats", "lh_stats_eval", "lh_get_step_stats", "lh_set_gradient", "lh_ppt_table",
             "lh_fno_create", "lh_fno_destroy", "lh_fno_param_count", "lh_fno_set_params",
             "lh_fno_get_params", "lh_fno_forward", "lh_fno_loss_grad", "lh_fno_set_data", "lh_fno_train"]

@@ -264,7 +264,8 @@ struct lh_ctx {
     RadArgs* rargs;      // [0]: solver, [1]: single RHS
     RadCtl* rctl;        // [0]: solver, [1]: single RHS
     hipGraphExec_t rgraph;
-    RadPlan rplan;       // variant of the RHS launch sequence (rgraph is captured with it)
+    RadPlan rplan;       // variant of the RHS launch sequence
+    int rplan_own;       // from the wisdom or lh_set_plan, else the default
     // per-step statistics
     double* omega;       // [Nω] ω (shared)
     double* st_ew;       // [Nω] energy weights (shared)
@@ -892,7 +893,8 @@ static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, DIn
 // The role of FFTW's wisdom in the reference (src/Utils.jl:84-108 imports it
 // before planning and exports it after): a context created for a shape with
 // wisdom takes the recorded plan without measuring; any other takes
-// RAD_DEFAULT_PLAN.  Process-wide, guarded by g_wisdom_mu.
+// RAD_DEFAULT_PLAN (with the tiles of rad_default_tiles).  Process-wide, guarded
+// by g_wisdom_mu.
 struct WisdomEntry {
     int n_to, n_r;
     RadPlan plan;
@@ -901,11 +903,11 @@ struct WisdomEntry {
 static std::mutex g_wisdom_mu;
 static std::vector<WisdomEntry> g_wisdom;
 
-static RadPlan wisdom_lookup(int n_to, int n_r) {
+static bool wisdom_lookup(int n_to, int n_r, RadPlan* p) {
     std::lock_guard<std::mutex> lk(g_wisdom_mu);
     for (const WisdomEntry& w : g_wisdom)
-        if (w.n_to == n_to && w.n_r == n_r) return w.plan;
-    return RAD_DEFAULT_PLAN;
+        if (w.n_to == n_to && w.n_r == n_r) return *p = w.plan, true;
+    return false;
 }
 
 static void wisdom_record(int n_to, int n_r, RadPlan p, double us) {
@@ -935,7 +937,8 @@ static int rad_setup(lh_ctx* c, const lh_desc* d) {
     HIPCK(hipMalloc(&c->partial, sizeof(double) * 3 * nr));
     HIPCK(hipMalloc(&c->rargs, sizeof(RadArgs) * 2));
     HIPCK(hipMalloc(&c->rctl, sizeof(RadCtl) * 2));
-    c->rplan = wisdom_lookup(d->n_to, d->n_r);
+    c->rplan = RAD_DEFAULT_PLAN;
+    c->rplan_own = wisdom_lookup(d->n_to, d->n_r, &c->rplan);
     DInst pw = base_inst(c);
     pw.e_scale = 1.0;  // the 1/Nto of the inverse transform is folded into the k→r contraction
     return upload(&c->pw, &pw, 1);
@@ -950,6 +953,12 @@ static void rad_ctl_init(RadCtl* h, const lh_rk_opts* o) {
     }
     for (int j = 0; j < 8; j++) h->perm[j] = j;
     h->status = LH_OK;
+}
+
+// The plan that the context's launches follow (rgraph is captured with it).
+static RadPlan rad_plan_run(const lh_ctx* c) {
+    if (c->rplan_own) return c->rplan;
+    return {c->rplan.fft, rad_default_tiles((c->d.grid_kind == LH_GRID_ENV ? 2 : 1) * c->d.n_to, c->d.n_r)};
 }
 
 static RadArgs rad_args(const lh_ctx* c, int slot) {
@@ -1019,7 +1028,7 @@ static int rad_solve(lh_ctx* c, const lh_rk_opts* o, bool want_saves, hipStream_
     h.rhs_evals = 1;
     hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, a, h, c->rargs);
     HIPCK(hipMemcpyAsync(c->Y, c->Yin, sizeof(double2) * (size_t)c->n_state, hipMemcpyDeviceToDevice, s));
-    rad_rhs_dispatch(c->rplan, c->d.grid_kind == LH_GRID_ENV, n_to, n_r, c->rargs, tw, -1, s);  // PreconStepper init: k1 = fbar(y0)
+    rad_rhs_dispatch(rad_plan_run(c), c->d.grid_kind == LH_GRID_ENV, n_to, n_r, c->rargs, tw, -1, s);  // PreconStepper init: k1 = fbar(y0)
     HIPCK(hipGetLastError());
     HIPCK(hipMemcpyAsync(&h, c->rctl, sizeof(h), hipMemcpyDeviceToHost, s));
     HIPCK(hipStreamSynchronize(s));
@@ -1030,7 +1039,7 @@ static int rad_solve(lh_ctx* c, const lh_rk_opts* o, bool want_saves, hipStream_
     if (!h.done && !c->rgraph) {
         hipGraph_t g = nullptr;
         HIPCK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        rad_step_dispatch(c->rplan, c->d.grid_kind == LH_GRID_ENV, n_to, n_r, c->rargs, tw, s);
+        rad_step_dispatch(rad_plan_run(c), c->d.grid_kind == LH_GRID_ENV, n_to, n_r, c->rargs, tw, s);
         hipError_t e1 = hipGetLastError();
         hipError_t e2 = hipStreamEndCapture(s, &g);
         if (e1 != hipSuccess || e2 != hipSuccess || !g) {
@@ -1290,7 +1299,7 @@ int lh_rhs_device(lh_ctx* c, void* nl_dev, const void* Ew_dev, double z, void* s
         rad_ctl_init(&one.h, nullptr);
         const bool env = c->d.grid_kind == LH_GRID_ENV;
         if (env) hipLaunchKernelGGL(rad_set, dim3(1), dim3(64), 0, s, one.a, one.h, c->rargs + 1);
-        rad_rhs_dispatch(c->rplan, env, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s, &one);
+        rad_rhs_dispatch(rad_plan_run(c), env, c->d.n_to, c->d.n_r, c->rargs + 1, tw, -1, s, &one);
     } else {
         DInst in = base_inst(c);
         in.rhs_in = (const double2*)Ew_dev;
@@ -2005,15 +2014,23 @@ int lh_set_plan(lh_ctx* c, const lh_plan* p) {
     if (!c || !p || c->d.transform != LH_TRANS_RADIAL) return LH_E_ARG;
     const RadPlan np = {p->fft_radix_plan, p->gemm_tiles};
     if (!rad_plan_ok(np)) return LH_E_ARG;
-    if (np.fft != c->rplan.fft || np.mt != c->rplan.mt) {
+    const RadPlan run = rad_plan_run(c);
+    if (np.fft != run.fft || np.mt != run.mt) {
         HIPCK(hipSetDevice(c->device));
         HIPCK(hipStreamSynchronize(c->stream));
         if (c->rgraph) {  // captured with the old plan
             (void)hipGraphExecDestroy(c->rgraph);
             c->rgraph = nullptr;
         }
-        c->rplan = np;
     }
+    c->rplan = np;
+    c->rplan_own = 1;
+    return LH_OK;
+}
+
+int lh_plan_tiles(const lh_ctx* c, int* tiles) {
+    if (!c || !tiles || c->d.transform != LH_TRANS_RADIAL) return LH_E_ARG;
+    *tiles = rad_plan_run(c).mt;
     return LH_OK;
 }
 

@@ -580,14 +580,16 @@ __global__ __launch_bounds__(64) void rad_set(RadArgs a, RadCtl h, RadArgs* ap) 
     *a.ctl = h;
 }
 
-// MFMA tiles per wave along t: the plan's, halved while the grid leaves half the
-// CUs without a workgroup (a wave with more tiles loads less per product).  Same
-// products in the same order, so the same bits.  µs per GEMM with 2 tiles / 1,
-// workgroups at 2 tiles: Nto × Nr = 2048 × 64 (32) 6.4/4.5, 4096 × 64 (64) 7.3/5.6,
-// 2048 × 128 (64) 9.5/7.4, 8192 × 64 (128) 7.6/6.0, 2048 × 256 (128) 15.7/12.2;
-// 4096 × 192 (192) 13.9/15.3, 8192 × 128 (256) 10.2/11.7, 8192 × 256 (512) 28.1/31.6.
-static int rad_tiles(const RadPlan& p, int rows, int n_r) {
-    int mt = p.mt;
+// MFMA tiles per wave along t of a context that has no plan of its own: the
+// default plan's, halved while the grid leaves half the CUs without a workgroup
+// (a wave with more tiles loads less per product).  Same products in the same
+// order, so the same bits.  A plan from the wisdom or lh_set_plan runs as it is.
+// µs per GEMM with 2 tiles / 1, workgroups at 2 tiles: Nto × Nr = 2048 × 64 (32)
+// 6.4/4.5, 4096 × 64 (64) 7.3/5.6, 2048 × 128 (64) 9.5/7.4, 8192 × 64 (128)
+// 7.6/6.0, 2048 × 256 (128) 15.7/12.2; 4096 × 192 (192) 13.9/15.3, 8192 × 128
+// (256) 10.2/11.7, 8192 × 256 (512) 28.1/31.6.
+static int rad_default_tiles(int rows, int n_r) {
+    int mt = RAD_DEFAULT_PLAN.mt;
     while (mt > 1 && (rows / (32 * mt)) * (n_r / 64) <= 128) mt /= 2;
     return mt;
 }
@@ -645,7 +647,7 @@ static void rad_run_env(bool step, const RadArgs* a, const double2* tw, int n_r,
 template <int NO>
 static void rad_run_env_mt(const RadPlan& p, bool step, const RadArgs* a, const double2* tw, int n_r, int stage,
                            hipStream_t s) {
-    switch (rad_tiles(p, 2 * NO, n_r)) {
+    switch (p.mt) {
         case 1: rad_run_env<NO, 1>(step, a, tw, n_r, stage, s); break;
         case 4: rad_run_env<NO, 4>(step, a, tw, n_r, stage, s); break;
         default: rad_run_env<NO, 2>(step, a, tw, n_r, stage, s); break;
@@ -670,7 +672,7 @@ static void rad_run(bool step, const RadArgs* a, const double2* tw, int n_to, in
 template <int MO, int MC, int PLAN>
 static void rad_run_mt(const RadPlan& p, bool step, const RadArgs* a, const double2* tw, int n_to, int n_r, int stage,
                        hipStream_t s, const RadOne* one) {
-    switch (rad_tiles(p, n_to, n_r)) {
+    switch (p.mt) {
         case 1: rad_run<MO, MC, PLAN, 1>(step, a, tw, n_to, n_r, stage, s, one); break;
         case 4: rad_run<MO, MC, PLAN, 4>(step, a, tw, n_to, n_r, stage, s, one); break;
         default: rad_run<MO, MC, PLAN, 2>(step, a, tw, n_to, n_r, stage, s, one); break;

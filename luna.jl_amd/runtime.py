@@ -46,6 +46,13 @@ class Context:
         p.fft_radix_plan, p.gemm_tiles = value
         _capi.check(_capi.lib().lh_set_plan(self.handle, C.byref(p)), "lh_set_plan")
 
+    @property
+    def plan_tiles(self):
+        """MFMA tiles that the launches run with (``lh_plan_tiles``)."""
+        n = C.c_int(0)
+        _capi.check(_capi.lib().lh_plan_tiles(self.handle, C.byref(n)), "lh_plan_tiles")
+        return n.value
+
     def autotune(self, Ew=None, reps=10):
         """Times every plan on one RHS of ``Ew`` (zero field if None) and
         installs the fastest; returns [(fft_radix_plan, gemm_tiles, µs per RHS,
