@@ -9,7 +9,8 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", n) for n in ("lh_kernels.hip", "lh_gang_field.hip", "lh_gang_raman.hip",
-                                                "lh_gang_env.hip", "lh_gang_dense.hip", "lh_solo.hip", "lh_fno.hip", "lh_ppt.hip")]
+                                                "lh_gang_env.hip", "lh_gang_dense.hip", "lh_solo.hip", "lh_solo_8192.hip",
+                                                "lh_fno.hip", "lh_ppt.hip")]
 OUT_DIR = os.path.join(HERE, "_build")
 OUT = os.path.join(OUT_DIR, "libluna_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -27,8 +28,9 @@ FLAGS = [
 # around its series; hoisting the FP64 constants of their exponentials and powers
 # out of it costs registers that then spill (gangs: 22 to 59 VGPRs against none,
 # 5 % of a propagation at Nto = 8192; z-dependent fills: 71 against none; PPT:
-# 126 VGPRs against 76).
+# 126 VGPRs against 76).  One solver is faster with it (lh_solo_8192.hip).
 LOOP_FLAGS = ["-mllvm", "-disable-machine-licm"]
+LOOP_FILES = ("lh_gang", "lh_solo.hip", "lh_ppt")
 
 H5_SRC = os.path.join(HERE, "csrc", "lh_h5.c")
 H5_OUT = os.path.join(OUT_DIR, "libluna_h5.so")
@@ -59,7 +61,7 @@ def build(verbose=False):
     os.makedirs(OUT_DIR, exist_ok=True)
     tag = f".tmp{os.getpid()}"
     objs = [os.path.join(OUT_DIR, os.path.basename(s).replace(".hip", ".o") + tag) for s in SRCS]
-    procs = [subprocess.Popen([HIPCC] + FLAGS + (LOOP_FLAGS if any(k in s for k in ("lh_gang", "lh_solo", "lh_ppt")) else []) + ["-c", "-o", o, s], stdout=subprocess.PIPE,
+    procs = [subprocess.Popen([HIPCC] + FLAGS + (LOOP_FLAGS if any(k in s for k in LOOP_FILES) else []) + ["-c", "-o", o, s], stdout=subprocess.PIPE,
                               stderr=subprocess.PIPE, text=True) for s, o in zip(SRCS, objs)]
     failed = []
     for p, s in zip(procs, SRCS):

@@ -1,4 +1,4 @@
-// lh_solo.h -- the launch of lh_solo.hip.
+// lh_solo.h -- the launches of lh_solo.hip and lh_solo_8192.hip.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -10,3 +10,4 @@ struct DInst;
 // 4096 points.  tw: the twiddle table of the single-workgroup transforms.  False:
 // no such kernel.
 bool launch_solo(int cls, int n, const DInst* d, const double2* tw, hipStream_t s, bool zdep, bool raman);
+void launch_solo_8192(int n, const DInst* d, const double2* tw, hipStream_t s);  // constant fill, Nto = 8192
