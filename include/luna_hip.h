@@ -388,6 +388,16 @@ int lh_get_step_stats(lh_ctx *ctx, double *rec, int capacity, int *n);
  * 32768), with the number of instances in each.  nclass must be >= 8. */
 int lh_last_launch_times(double *ms, int *n_inst, int nclass);
 
+/* Which kernels the last batch ran on, per grid-size class as above: a sum of
+ * LH_KIND_*, 0 for a class without instances.  nclass must be >= 8. */
+enum {
+    LH_KIND_GANG = 1,       /* gangs of four workgroups                        */
+    LH_KIND_GANG_DENSE = 2, /* the same, two workgroups per CU                 */
+    LH_KIND_ALONE = 4,      /* one workgroup per instance                      */
+    LH_KIND_RADIAL = 8      /* launch sequence per step                        */
+};
+int lh_last_launch_kinds(int *kinds, int nclass);
+
 /* Page-locked host memory for the states and saves a sweep copies back (no
  * counterpart in the reference, whose arrays live in host memory already):
  * device-to-host copies into it run at DMA speed and touch no unmapped pages.

@@ -12,6 +12,7 @@ import numpy as np
 (LH_OK, LH_E_ARG, LH_E_HIP, LH_E_PPT_RANGE, LH_E_REPEAT_LIMIT, LH_E_NONFINITE, LH_E_NOMEM, LH_E_NODEVICE,
  LH_E_MAXSTEPS, LH_E_STOPPED, LH_E_TOO_LARGE, LH_E_HOST_WAIT) = range(12)
 LH_NOALLOC_SCRATCH_BYTES = 1536 * 1024
+LH_KIND_GANG, LH_KIND_GANG_DENSE, LH_KIND_ALONE, LH_KIND_RADIAL = 1, 2, 4, 8
 LH_GRID_REAL, LH_GRID_ENV = 0, 1
 LH_TRANS_MODEAVG, LH_TRANS_RADIAL = 0, 1
 LH_KERR_NONE, LH_KERR_FIELD, LH_KERR_ENV = 0, 1, 2
@@ -208,6 +209,7 @@ def lib():
     L.lh_batch_solve_resident.argtypes = [C.POINTER(C.c_void_p), C.c_int, C.POINTER(LhRkOpts), C.c_int,
                                           C.POINTER(LhStats)]
     L.lh_last_launch_times.argtypes = [_dp, C.POINTER(C.c_int), C.c_int]
+    L.lh_last_launch_kinds.argtypes = [C.POINTER(C.c_int), C.c_int]
     L.lh_host_alloc.argtypes = [C.c_size_t, C.POINTER(C.c_void_p)]
     L.lh_host_free.argtypes = [C.c_void_p]
     L.lh_solve_noalloc.argtypes = [C.c_void_p, C.c_void_p, C.POINTER(LhRkOpts), C.c_void_p, _dp,
@@ -240,7 +242,7 @@ def lib():
 
 EXPORTED = ["lh_strerror", "lh_device_count", "lh_create", "lh_destroy", "lh_rhs",
             "lh_rhs_device", "lh_ctx_status", "lh_solve", "lh_solve_stream", "lh_batch_solve", "lh_batch_solve_opts", "lh_set_state",
-            "lh_batch_solve_resident", "lh_get_state", "lh_get_saves", "lh_last_launch_times",
+            "lh_batch_solve_resident", "lh_get_state", "lh_get_saves", "lh_last_launch_times", "lh_last_launch_kinds",
             "lh_host_alloc", "lh_host_free", "lh_solve_noalloc",
             "lh_get_plan", "lh_set_plan", "lh_plan_tiles", "lh_autotune", "lh_wisdom_export", "lh_wisdom_import", "lh_wisdom_forget",
             "lh_set_step_stats", "lh_stats_eval", "lh_get_step_stats", "lh_set_gradient", "lh_ppt_table",

@@ -310,9 +310,10 @@ static unsigned char* g_scratch[64] = {nullptr};
 // The word of each GPU that its solvers change as they get on (GangCtl::beat).
 static __device__ unsigned beat;
 static unsigned* g_beat[64] = {nullptr};
-// HIP-event durations of the last resident batch, per size class
+// HIP-event durations of the last resident batch and its kernels (LH_KIND_*), per size class
 static float g_last_ms[8] = {0};
 static int g_last_n[8] = {0};
+static int g_last_kind[8] = {0};
 
 #define HIPCK(x)                                                                     \
     do {                                                                             \
@@ -1758,10 +1759,15 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         st = LH_E_HIP;
     if (hipStreamSynchronize(s0) != hipSuccess && !st) st = LH_E_HIP;
     float cls_ms[LH_NCLASS] = {0};
-    int cls_n[LH_NCLASS] = {0};
+    int cls_n[LH_NCLASS] = {0}, cls_kind[LH_NCLASS] = {0};
     for (int c = 0; c < NG; c++) {
         float ms = 0.0f;
         cls_n[c % LH_NCLASS] += count[c];
+        if (count[c])
+            cls_kind[c % LH_NCLASS] |= c == LH_CLASS_RADIAL         ? LH_KIND_RADIAL
+                                       : c >= V_ZDEP * LH_NCLASS    ? LH_KIND_ALONE
+                                       : dense[c]                   ? LH_KIND_GANG_DENSE
+                                                                    : LH_KIND_GANG;
         if (!st && t0[c] && t1[c] && hipEventElapsedTime(&ms, t0[c], t1[c]) == hipSuccess && ms > cls_ms[c % LH_NCLASS])
             cls_ms[c % LH_NCLASS] = ms;
         if (t0[c]) (void)hipEventDestroy(t0[c]);
@@ -1771,6 +1777,7 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     for (int c = 0; c < LH_NCLASS && !st; c++) {
         g_last_ms[c] = cls_ms[c];
         g_last_n[c] = cls_n[c];
+        g_last_kind[c] = cls_kind[c];
     }
     if (ready) (void)hipEventDestroy(ready);
     (void)hipFree(dblk);
@@ -1993,11 +2000,17 @@ int lh_get_step_stats(lh_ctx* c, double* rec, int capacity, int* n) {
 }
 
 int lh_last_launch_times(double* ms, int* n_inst, int nclass) {
-    if (!ms || !n_inst || nclass < LH_NCLASS) return LH_E_ARG;  // LH_NCLASS = 6
+    if (!ms || !n_inst || nclass < LH_NCLASS) return LH_E_ARG;
     for (int c = 0; c < LH_NCLASS; c++) {
         ms[c] = g_last_ms[c];
         n_inst[c] = g_last_n[c];
     }
+    return LH_OK;
+}
+
+int lh_last_launch_kinds(int* kinds, int nclass) {
+    if (!kinds || nclass < LH_NCLASS) return LH_E_ARG;
+    for (int c = 0; c < LH_NCLASS; c++) kinds[c] = g_last_kind[c];
     return LH_OK;
 }
 

@@ -404,3 +404,11 @@ def last_launch_times():
     n = (C.c_int * k)()
     _capi.check(_capi.lib().lh_last_launch_times(ms, n, k), "lh_last_launch_times")
     return {_capi.CLASS_NAMES[c]: (ms[c], n[c]) for c in range(k) if n[c] > 0}
+
+
+def last_launch_kinds():
+    """{n_to: sum of LH_KIND_*} of the last batch's kernels."""
+    k = len(_capi.CLASS_NAMES)
+    kinds = (C.c_int * k)()
+    _capi.check(_capi.lib().lh_last_launch_kinds(kinds, k), "lh_last_launch_kinds")
+    return {_capi.CLASS_NAMES[c]: kinds[c] for c in range(k) if kinds[c]}

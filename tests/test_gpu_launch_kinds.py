@@ -1,0 +1,57 @@
+"""Which kernels a batch runs on: the batches of test_gpu_gang_dense.py,
+test_gpu_solo.py and test_gpu_solo_kinds.py reach the kernels they are about."""
+import pytest
+
+import test_gpu_gang_dense
+import test_gpu_solo_kinds
+
+pytestmark = pytest.mark.gpu
+
+
+def kinds_of(holders, fields, opts):
+    from luna_jl_amd import runtime
+    rb = runtime.ResidentBatch([runtime.Context(h) for h in holders], fields)
+    assert all(s.status == 0 for s in rb.solve(opts, want_saves=False))
+    return runtime.last_launch_kinds()
+
+
+@pytest.mark.parametrize("n", [177, 300])
+def test_uneven(pkg, capi, n):
+    print(f"case: kinds of an uneven batch of {n}", flush=True)
+    from luna_jl_amd import configs
+    insts = test_gpu_gang_dense._batch(configs, n)
+    k = kinds_of([c.holder for c in insts], [c.Ew0 for c in insts], capi.rk_opts(2e-4, save_n=2, init_dz=2e-4))
+    assert {k[c] for c in (4096, 8192, 16384)} == {capi.LH_KIND_GANG_DENSE}
+    assert {v for c, v in k.items() if str(c).startswith("env")} == {capi.LH_KIND_GANG}
+
+
+@pytest.mark.parametrize("trange,n,nonlinear", [(0.25e-12, 200, True), (0.5e-12, 256, True), (1e-12, 257, True),
+                                                (0.25e-12, 256, False)])
+def test_even_field(pkg, capi, trange, n, nonlinear):
+    print(f"case: kinds of an even batch {trange} {n}", flush=True)
+    from luna_jl_amd import configs
+    kw = {} if nonlinear else dict(kerr=False, plasma=False)
+    c = configs.capillary_instance(energy=80e-6, pressure=1.0, trange=trange, flength=0.1, ppt_n=2 ** 12, **kw)
+    E0 = [c.Ew0 * (1.0 + 1e-4 * (i % 7)) for i in range(n)]
+    assert list(kinds_of([c.holder] * n, E0, capi.rk_opts(2e-3, save_n=2, init_dz=2e-3)).values()) == [capi.LH_KIND_ALONE]
+
+
+@pytest.mark.parametrize("make,n", [(lambda: test_gpu_solo_kinds._molecular(0.25e-12), 200),
+                                    (lambda: test_gpu_solo_kinds._molecular(0.5e-12), 256),
+                                    (test_gpu_solo_kinds._envelope, 257)])
+def test_even_kinds(pkg, capi, make, n):
+    print(f"case: kinds of an even batch of {n}", flush=True)
+    holder, E0, _, dz = make()
+    assert list(kinds_of([holder] * n, [E0] * n, capi.rk_opts(dz, save_n=2, init_dz=dz)).values()) == [capi.LH_KIND_ALONE]
+
+
+def test_others(pkg, capi):
+    print("case: kinds of single instances", flush=True)
+    from luna_jl_amd import configs
+    c = configs.capillary_instance(trange=0.25e-12, flength=0.1, ppt_n=2 ** 12)
+    z = test_gpu_solo_kinds._molecular(0.25e-12)
+    opts = capi.rk_opts(1e-3, save_n=2, init_dz=1e-3)
+    assert kinds_of([c.holder], [c.Ew0], opts) == {4096: capi.LH_KIND_GANG}
+    assert kinds_of([c.holder, z[0]], [c.Ew0, z[1]], opts) == {4096: capi.LH_KIND_GANG}
+    r = configs.radial_instance(flength=0.1, energy=50e-6, propz=-0.05, R=1.5e-3, N=64, trange=0.3e-12)
+    assert kinds_of([r.holder, c.holder], [r.Ew0, c.Ew0], opts) == {"radial": capi.LH_KIND_RADIAL, 4096: capi.LH_KIND_GANG}
