@@ -33,7 +33,9 @@
 #include <string.h>
 
 #include <algorithm>
+#include <functional>
 #include <mutex>
+#include <queue>
 #include <string>
 #include <time.h>
 #include <vector>
@@ -805,29 +807,35 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
 }
 
 // Whether the constant-fill instances of a batch run on one workgroup each
-// (lh_solo.hip) instead of on gangs.  Both ways are priced with the estimated
-// lengths of their runs: alone, the slowest instance or the work over the CUs
-// decides; on gangs the work does, and a tail of a tenth or more.  µs per
-// right-hand side: one workgroup 23.4, 37.4, 63.7 at Nto = 4096, 8192, 16384;
+// (lh_solo_kernel.h) instead of on gangs.  Both ways are priced with the
+// estimated lengths of their runs, dealt longest first to the places there are:
+// 256 workgroups alone, 64 gangs or 128 dense ones; gangs share the chip between
+// classes, which costs a tenth or more of their work.  Equal instances come in
+// rounds: 65 to 128 of them occupy 64 gangs as long as 128 do.  µs per
+// right-hand side, one workgroup 23.4, 37.4, 63.7 at Nto = 4096, 8192, 16384;
 // gangs, per instance on the whole chip, 0.275, 0.31, 0.455 at one workgroup per
 // CU and 0.241, 0.26, 0.382 on dense kernels; the other entries of solo_price
-// likewise (with a Raman response; the envelope grid of 4096 points).  Grids that
-// have no entry are faster on gangs at every number of instances.  256 equal instances: 3.8, 6.1,
-// 10.4 ms alone against 10.1, 10.9, 16.0 on gangs; sweeps whose longest run is
-// twice the mean: 51 against 40 ms with 256 points, 26 against 34 with 384 (half
-// as long), 53 against 76 with 512.  The rule depends on the batch alone, so a
-// batch gives the same bits every time; the two ways agree to rounding.
+// likewise (with a Raman response; the envelope grid of 4096 points).  Field
+// grids without an entry, and envelope grids of 8192 points and more, have no
+// kernel for one workgroup: at 16 to 512 equal instances gangs took 0.2 to 0.97
+// of the time that one did when it had.
+// Equal instances, ms alone / on gangs: Nto = 4096, 72 3.3/5.9; 8192, 72 5.3/6.5;
+// 16384, 72 9.8/9.7; Raman 4096, 72 12.2/14.7, 8192, 72 21.9/17.9, 176 24.2/28.5;
+// envelope 4096, 72 10.5/9.0, 256 of each field grid 3.8, 6.1, 10.4 against 10.1,
+// 10.9, 16.0.  Sweeps whose longest run is twice the mean: 51 against 40 ms with
+// 256 points, 26 against 34 with 384 (half as long), 53 against 76 with 512.  The
+// rule depends on the batch alone, so a batch gives the same bits every time.
 struct SoloPrice {
     double alone, gang, dense;  // µs: alone per right-hand side, on gangs per instance
 };
 static bool solo_price(const lh_ctx* c, SoloPrice* p) {
     if (c->d.transform != LH_TRANS_MODEAVG || c->zg_on) return false;
     const int cls = ctx_class(c);
-    if (cls == LH_CLASS_ENV4096) return *p = {57.5, 0.341, 0.341}, true;
+    if (cls == LH_CLASS_ENV4096) return *p = {53.5, 0.341, 0}, true;
     if (c->d.grid_kind != LH_GRID_REAL) return false;
     if (c->d.raman) {
-        if (cls == LH_CLASS_8192) return *p = {103.7, 0.511, 0.511}, true;
-        if (cls == LH_CLASS_4096) return *p = {48.4, 0.404, 0.404}, true;
+        if (cls == LH_CLASS_8192) return *p = {90.0, 0.511, 0}, true;
+        if (cls == LH_CLASS_4096) return *p = {48.4, 0.404, 0}, true;
         return false;
     }
     if (cls == LH_CLASS_16384) return *p = {63.7, 0.455, 0.382}, true;
@@ -835,27 +843,42 @@ static bool solo_price(const lh_ctx* c, SoloPrice* p) {
     if (cls == LH_CLASS_4096) return *p = {23.4, 0.275, 0.241}, true;
     return false;
 }
-static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
-    const bool dense = n > LG_DENSE_ABOVE;
-    double longest = 0.0, alone = 0.0, gangs = 0.0;
-    int m = 0, zero = 0;
-    SoloPrice p;
-    for (int pass = 0; pass < 2; pass++) {
-        for (int i = 0; i < n; i++) {
-            if (!solo_price(ctxs[i], &p)) continue;
-            double w = solve_cost(ctxs[i], op[i]) / class_us(ctx_class(ctxs[i]));
-            if (pass == 0) {
-                m++;
-                zero += (w == 0.0);
-                continue;
-            }
-            if (zero == m) w = 1.0;  // linear runs: equal lengths
-            longest = std::max(longest, w * p.alone);
-            alone += w * p.alone / LG_MAX_WG;
-            gangs += w * (dense ? p.dense : p.gang);
+// When the last of these runs ends, dealt longest first to so many places.
+static double dealt(std::vector<double>& w, int places) {
+    std::sort(w.begin(), w.end(), std::greater<double>());
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
+    double end = 0.0;
+    for (double x : w) {
+        if ((int)free_at.size() == places) {
+            x += free_at.top();
+            free_at.pop();
         }
+        free_at.push(x);
+        end = std::max(end, x);
     }
-    return m > 0 && std::max(longest, alone) < 1.1 * gangs;
+    return end;
+}
+static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
+    constexpr int GANGS = LG_MAX_WG / LG_G;
+    std::vector<double> cost;
+    std::vector<SoloPrice> price;
+    SoloPrice p;
+    for (int i = 0; i < n; i++)
+        if (solo_price(ctxs[i], &p)) {
+            cost.push_back(solve_cost(ctxs[i], op[i]) / class_us(ctx_class(ctxs[i])));
+            price.push_back(p);
+        }
+    if (cost.empty()) return false;
+    if (*std::max_element(cost.begin(), cost.end()) == 0.0) cost.assign(cost.size(), 1.0);  // linear runs: equal lengths
+    std::vector<double> alone, gang, dense;
+    double work = 0.0;
+    for (size_t i = 0; i < cost.size(); i++) {
+        const bool d = n > LG_DENSE_ABOVE && price[i].dense > 0;
+        alone.push_back(cost[i] * price[i].alone);
+        (d ? dense : gang).push_back(cost[i] * (d ? 2 * GANGS * price[i].dense : GANGS * price[i].gang));
+        work += cost[i] * (d ? price[i].dense : price[i].gang);
+    }
+    return dealt(alone, LG_MAX_WG) < std::max({1.1 * work, dealt(gang, GANGS), dealt(dense, 2 * GANGS)});
 }
 
 static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, bool alone, DInst* in,

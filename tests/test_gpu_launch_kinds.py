@@ -55,3 +55,20 @@ def test_others(pkg, capi):
     assert kinds_of([c.holder, z[0]], [c.Ew0, z[1]], opts) == {4096: capi.LH_KIND_GANG}
     r = configs.radial_instance(flength=0.1, energy=50e-6, propz=-0.05, R=1.5e-3, N=64, trange=0.3e-12)
     assert kinds_of([r.holder, c.holder], [r.Ew0, c.Ew0], opts) == {"radial": capi.LH_KIND_RADIAL, 4096: capi.LH_KIND_GANG}
+
+
+@pytest.mark.parametrize("make,most", [(4096, 64), (8192, 64), (16384, 127), ("N2", 64), ("env", 128)])
+def test_even_batches_on_each_side(pkg, capi, make, most):
+    """Equal instances stay on gangs while those take them in one round (in two
+    where a round is short enough), and go to one workgroup each above."""
+    print(f"case: kinds at {most} and {most + 1} equal instances, {make}", flush=True)
+    from luna_jl_amd import configs
+    if make == "N2":
+        holder, E0, _, dz = test_gpu_solo_kinds._molecular(0.25e-12)
+    elif make == "env":
+        holder, E0, _, dz = test_gpu_solo_kinds._envelope()
+    else:
+        c = configs.capillary_instance(trange={4096: 0.25e-12, 8192: 0.5e-12, 16384: 1e-12}[make], flength=0.1, ppt_n=2 ** 12)
+        holder, E0, dz = c.holder, c.Ew0, 2e-3
+    for n, kind in [(most, capi.LH_KIND_GANG), (most + 1, capi.LH_KIND_ALONE)]:
+        assert list(kinds_of([holder] * n, [E0] * n, capi.rk_opts(dz, save_n=2, init_dz=dz)).values()) == [kind], n
