@@ -222,9 +222,16 @@ int lh_solve_stream(lh_ctx *ctx, double *Ew_inout, const lh_rk_opts *opts, lh_ou
 
 /* Batched solve: n independent instances (each its own grid, constants, step
  * size control and status) in one persistent launch per grid class, a gang of
- * four workgroups per instance (z-dependent fills and large even batches:
- * one workgroup, whose results agree with a gang's to rounding),
- * the expensive instances first.  Radial contexts (whose one instance fills the GPU)
+ * four workgroups per instance, the expensive instances first, or one workgroup
+ * (z-dependent fills; and even batches of more than some 64 instances, where
+ * that is faster: lh_last_launch_kinds tells).  Solved by itself an instance
+ * runs on a gang, so it gets the same bits from a batch on gangs, and others
+ * from an even batch: the spectra then agree to 5e-13, the fields to 3e-11;
+ * with a first step so small that its error estimate is rounding noise, as the
+ * default 1e-4 m is, that noise sets the next step, and the spectra agree to
+ * 5e-9, the fields to 1.4e-6 (256 equal propagations of 0.05 to 0.5 m in each
+ * class, against one).  A batch repeated gives the same bits.
+ * Radial contexts (whose one instance fills the GPU)
  * are solved one after another by a graph-replayed per-step launch sequence.
  * Replaces the per-point loop of Scans.runscan src/Scans.jl:275-430.
  * Ew_inout[i]: instance i's field; saves[i] may be NULL; stats[i] per instance.

@@ -824,7 +824,8 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
 // envelope 4096, 72 10.5/9.0, 256 of each field grid 3.8, 6.1, 10.4 against 10.1,
 // 10.9, 16.0.  Sweeps whose longest run is twice the mean: 51 against 40 ms with
 // 256 points, 26 against 34 with 384 (half as long), 53 against 76 with 512.  The
-// rule depends on the batch alone, so a batch gives the same bits every time.
+// rule depends on the batch alone, so a batch gives the same bits every time;
+// what the two ways differ by is with lh_batch_solve in luna_hip.h.
 struct SoloPrice {
     double alone, gang, dense;  // µs: alone per right-hand side, on gangs per instance
 };

@@ -72,3 +72,28 @@ def test_even_batches_on_each_side(pkg, capi, make, most):
         holder, E0, dz = c.holder, c.Ew0, 2e-3
     for n, kind in [(most, capi.LH_KIND_GANG), (most + 1, capi.LH_KIND_ALONE)]:
         assert list(kinds_of([holder] * n, [E0] * n, capi.rk_opts(dz, save_n=2, init_dz=dz)).values()) == [kind], n
+
+
+@pytest.mark.parametrize("init_dz", [1e-4, 2e-3])
+def test_even_batch_against_one(pkg, capi, init_dz):
+    """An instance of an even batch (one workgroup) and the same one solved by
+    itself (a gang) take the same steps and agree to the propagation tests' 1e-6
+    in spectral energy, also with the default first step, whose error estimate is
+    rounding noise and sets the next step."""
+    print(f"case: even batch against one, first step {init_dz}", flush=True)
+    import numpy as np
+    from luna_jl_amd import configs, runtime
+    c = configs.capillary_instance(energy=80e-6, pressure=1.0, trange=0.5e-12, flength=0.1, ppt_n=2 ** 12)
+    opts = capi.rk_opts(0.1, save_n=5, init_dz=init_dz)
+    ctxs = [runtime.Context(c.holder) for _ in range(65)]
+    states, saves, _, st = runtime.batch_solve(ctxs, [c.Ew0] * 65, opts)
+    assert runtime.last_launch_kinds() == {8192: capi.LH_KIND_ALONE}
+    E, sv, _, s = ctxs[0].solve(c.Ew0, opts)
+    assert runtime.last_launch_kinds() == {8192: capi.LH_KIND_GANG}
+
+    def err(a, b):
+        a, b = np.abs(a) ** 2, np.abs(b) ** 2
+        return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+    assert (st[64].steps, st[64].rejected) == (s.steps, s.rejected)
+    assert err(states[64], E) <= 1e-6 and err(saves[64], sv) <= 1e-6
