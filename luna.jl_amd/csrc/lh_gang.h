@@ -794,30 +794,7 @@ __device__ __forceinline__ void g_zg_refresh(const DInst& in, SM& sm, int h, dou
                                              double& rho, double& kfac) {
     using Z = GSizes<KIND, M>;
     const int tid = fresh_tid();
-    if (tid < 64) {
-        const double p = zg_pressure(in, z);
-        const double r = cspline_uniform(gl(in.zd), in.zd_n, gl(in.zd)[0].x, gl(in.zd)[in.zd_n - 1].x, p);
-        const double a = in.ztaper ? zg_radius(in, z) : 0.0;
-        const int j = min(tid, 8);
-        const double* f = gl(in.zfd) + 4 * j;
-        const double sc = sqrt(1 + f[1] * r);
-        double2 nwj = make_double2(f[2], f[3]);
-        if (in.ztaper) {
-            const double* t = gl(in.zfdt) + 3 * j;
-            nwj = zg_nwg_taper(in, t[0], make_double2(t[1], t[2]), a);
-        }
-        double nr = zg_neff(in, sc * sc, nwj).x;
-        if (in.zg_model == 0 && nr < 1e-3) nr = 1e-3;
-        const double beta = f[0] / LH_CLIGHT * nr;
-        double acc = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) acc = fma(c_fd8[i], lane_value(beta, i), acc);
-        if (tid == 0) {
-            sm.zs[0] = r;
-            sm.zs[1] = acc / in.zfd_h;
-            sm.zs[2] = a;
-        }
-    }
+    if (tid < 64) zg_constants(in, sm.zs, z);
     __syncthreads();
     rho = sm.zs[0];
     const double b1 = sm.zs[1], a = sm.zs[2];

@@ -48,65 +48,6 @@
 
 static const long long LH_MAX_STEPS = 500000;  // default cap on step attempts per instance
 
-// exp(−2πi k/L) for the zero-padded Raman transforms: L up to LH_TWN from
-// the table; L = 2·LH_TWN gives even k from the table and odd k one more
-// factor exp(−2πi/L).
-template <int L>
-__device__ __forceinline__ double2 tw_frac(const TwLds& tw, int k) {
-    if constexpr (L <= LH_TWN) {
-        return tw_get(tw, k * (LH_TWN / L));
-    } else {
-        static_assert(L == 2 * LH_TWN, "tw_frac: L up to 2·LH_TWN");
-        double2 w = tw_get(tw, k >> 1);
-        if (k & 1) {
-            double sn, cs;
-            sincos(-6.283185307179586476925286766559 / (double)L, &sn, &cs);
-            w = cmul(w, make_double2(cs, sn));
-        }
-        return w;
-    }
-}
-
-// Unnormalised complex FFT of NO = 2·M points held in HBM (natural order, in
-// place in g); tmp: M points of HBM.  X[k] = E[k] + w^k O[k], X[k+M] =
-// E[k] − w^k O[k], with E, O the transforms of the even and odd samples and
-// w = exp(∓2πi/NO).  Starts and ends with a workgroup barrier.
-template <int M, bool INV, class Smem>
-__device__ __forceinline__ void fft_big(double2* g, double2* tmp, Smem& sm) {
-    const int tid = fresh_tid();
-    __syncthreads();
-    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j];
-    __syncthreads();
-    fft_lds<M, INV>(sm.buf, sm.tw);
-    for (int j = tid; j < M; j += LH_T) tmp[j] = sm.buf[pad(j)];
-    __syncthreads();
-    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j + 1];
-    __syncthreads();
-    fft_lds<M, INV>(sm.buf, sm.tw);
-    constexpr int TS = LH_TWN / (2 * M);
-    for (int k = tid; k < M; k += LH_T) {
-        double2 w = tw_get(sm.tw, k * TS);
-        if (INV) w.y = -w.y;
-        const double2 o = cmul(w, sm.buf[pad(k)]), e = tmp[k];
-        g[k] = cadd(e, o);
-        g[k + M] = csub(e, o);
-    }
-    __syncthreads();
-}
-
-// r2c post-step of a 2·NO-point real transform whose packed NO-point
-// transform Z is in HBM: X[k] = E + w^k O (as r2c_bin).
-template <int NO, class Smem>
-__device__ __forceinline__ double2 r2c_bin_big(const double2* Z, const Smem& sm, int k) {
-    double2 zk = Z[k == NO ? 0 : k];
-    double2 zc = cconj(Z[k == 0 ? 0 : NO - k]);
-    double2 E = cscal(0.5, cadd(zk, zc));
-    double2 d = csub(zk, zc);
-    double2 O = make_double2(0.5 * d.y, -(0.5 * d.x));
-    double2 w = (k == NO) ? make_double2(-1.0, 0.0) : tw_frac<2 * NO>(sm.tw, k);
-    return cadd(E, cmul(w, O));
-}
-
 // hω·δt on the big grid: h zero-padded to 2·NO reals, packed into NO complex
 // points in W, transformed, post-stepped into hwdt[0..NO].  One workgroup.
 template <int NO>

@@ -56,65 +56,6 @@ struct EpiStageFO {
     }
 };
 
-// exp(−2πi k/L) for the zero-padded Raman transforms: L up to LH_TWN from
-// the table; L = 2·LH_TWN gives even k from the table and odd k one more
-// factor exp(−2πi/L).
-template <int L>
-__device__ __forceinline__ double2 tw_frac(const TwLds& tw, int k) {
-    if constexpr (L <= LH_TWN) {
-        return tw_get(tw, k * (LH_TWN / L));
-    } else {
-        static_assert(L == 2 * LH_TWN, "tw_frac: L up to 2·LH_TWN");
-        double2 w = tw_get(tw, k >> 1);
-        if (k & 1) {
-            double sn, cs;
-            sincos(-6.283185307179586476925286766559 / (double)L, &sn, &cs);
-            w = cmul(w, make_double2(cs, sn));
-        }
-        return w;
-    }
-}
-
-// Unnormalised complex FFT of NO = 2·M points held in HBM (natural order, in
-// place in g); tmp: M points of HBM.  X[k] = E[k] + w^k O[k], X[k+M] =
-// E[k] − w^k O[k], with E, O the transforms of the even and odd samples and
-// w = exp(∓2πi/NO).  Starts and ends with a workgroup barrier.
-template <int M, bool INV, class Smem>
-__device__ __forceinline__ void fft_big(double2* g, double2* tmp, Smem& sm) {
-    const int tid = fresh_tid();
-    __syncthreads();
-    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j];
-    __syncthreads();
-    fft_lds<M, INV>(sm.buf, sm.tw);
-    for (int j = tid; j < M; j += LH_T) tmp[j] = sm.buf[pad(j)];
-    __syncthreads();
-    for (int j = tid; j < M; j += LH_T) sm.buf[pad(j)] = g[2 * j + 1];
-    __syncthreads();
-    fft_lds<M, INV>(sm.buf, sm.tw);
-    constexpr int TS = LH_TWN / (2 * M);
-    for (int k = tid; k < M; k += LH_T) {
-        double2 w = tw_get(sm.tw, k * TS);
-        if (INV) w.y = -w.y;
-        const double2 o = cmul(w, sm.buf[pad(k)]), e = tmp[k];
-        g[k] = cadd(e, o);
-        g[k + M] = csub(e, o);
-    }
-    __syncthreads();
-}
-
-// r2c post-step of a 2·NO-point real transform whose packed NO-point
-// transform Z is in HBM: X[k] = E + w^k O (as r2c_bin).
-template <int NO, class Smem>
-__device__ __forceinline__ double2 r2c_bin_big(const double2* Z, const Smem& sm, int k) {
-    double2 zk = Z[k == NO ? 0 : k];
-    double2 zc = cconj(Z[k == 0 ? 0 : NO - k]);
-    double2 E = cscal(0.5, cadd(zk, zc));
-    double2 d = csub(zk, zc);
-    double2 O = make_double2(0.5 * d.y, -(0.5 * d.x));
-    double2 w = (k == NO) ? make_double2(-1.0, 0.0) : tw_frac<2 * NO>(sm.tw, k);
-    return cadd(E, cmul(w, O));
-}
-
 // The convolution step of the zero-padded Raman transform (2·NO reals packed
 // into the NO-point transform Z in HBM): r2c post-step, ×hω·δt, and the c2r
 // pre-pack of the product, pairwise (k, NO − k) in place.
@@ -232,32 +173,7 @@ __device__ __forceinline__ void stage_prologue(const DInst& in, Smem& sm, const 
 template <class Smem>
 __device__ __forceinline__ void zg_refresh(const DInst& in, Smem& sm, double z, double& rho, double& kfac) {
     const int tid = fresh_tid();
-    if (tid < 64) {
-        const double p = zg_pressure(in, z);
-        const double r = cspline_uniform(gl(in.zd), in.zd_n, gl(in.zd)[0].x, gl(in.zd)[in.zd_n - 1].x, p);
-        // β1 = Modes.dispersion(mode, 1, ω0, z): β(ω) = ω/c·Re neff(mode, ω; z)
-        // with neff's own clamp (src/Capillary.jl:162-186)
-        const double a = in.ztaper ? zg_radius(in, z) : 0.0;
-        const int j = min(tid, 8);
-        const double* f = gl(in.zfd) + 4 * j;
-        const double sc = sqrt(1 + f[1] * r);
-        double2 nwj = make_double2(f[2], f[3]);
-        if (in.ztaper) {
-            const double* t = gl(in.zfdt) + 3 * j;
-            nwj = zg_nwg_taper(in, t[0], make_double2(t[1], t[2]), a);
-        }
-        double nr = zg_neff(in, sc * sc, nwj).x;
-        if (in.zg_model == 0 && nr < 1e-3) nr = 1e-3;
-        const double beta = f[0] / LH_CLIGHT * nr;
-        double acc = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) acc = fma(c_fd8[i], lane_value(beta, i), acc);
-        if (tid == 0) {
-            sm.zs[0] = r;
-            sm.zs[1] = acc / in.zfd_h;
-            sm.zs[2] = a;
-        }
-    }
+    if (tid < 64) zg_constants(in, sm.zs, z);
     __syncthreads();
     rho = sm.zs[0];
     const double b1 = sm.zs[1];
