@@ -15,7 +15,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -42,7 +41,11 @@ class HostPages {
         const uintptr_t e = ((uintptr_t)p + bytes) & ~(page - 1);
         while (a < e) {
             const uintptr_t b = std::min(e, (a + huge) & ~(huge - 1));
-            pieces.push_back({(char*)a, b - a});
+            try {
+                pieces.push_back({(char*)a, b - a});
+            } catch (...) {  // the rest is left to the copy
+                return;
+            }
             a = b;
         }
     }
@@ -57,7 +60,7 @@ class HostPages {
                         if (k >= pieces.size() || madvise(pieces[k].first, pieces[k].second, populate_write)) return;
                     }
                 });
-        } catch (const std::system_error&) {  // no more threads: what was started does it
+        } catch (...) {  // no more threads or memory: what was started does it
         }
     }
     void wait() {
@@ -108,7 +111,7 @@ static hipError_t copy_to_host(void* dst, const void* src, size_t bytes, int dev
         int begun = 0;
         try {
             for (int i = 1; i < LH_COPY_THREADS; i++, begun++) th.emplace_back(work, i);
-        } catch (const std::system_error&) {
+        } catch (...) {  // this thread does the rest
         }
         work(0);
         for (auto& t : th) t.join();
