@@ -26,13 +26,11 @@ static inline size_t lg_area_len(const lh_desc& d) {  // complex points of the e
     return 2 * lg_exchange_len(d) + 256 + (size_t)lg_points(d) / 2;
 }
 
-// Workgroups of a launch over n jobs that gets a share of the CUs: whole gangs
-// in equal numbers on the eight XCDs, one workgroup per CU, two of a dense kernel.
+// Workgroups of a launch over n jobs: whole gangs in equal numbers on the eight
+// XCDs, at most one workgroup per CU, two of a dense kernel.
 static constexpr int LG_MAX_WG = 256;        // one workgroup per CU
-static inline int lg_workgroups(int n, double share, bool dense) {
-    const int want = (LG_G * n + LG_MIN_WG - 1) / LG_MIN_WG * LG_MIN_WG;
-    int most = (int)(share * ((dense ? 2 : 1) * LG_MAX_WG / LG_MIN_WG) + 0.5) * LG_MIN_WG;
-    if (most < LG_MIN_WG) most = LG_MIN_WG;
+static inline int lg_workgroups(int n, bool dense) {
+    const int want = (LG_G * n + LG_MIN_WG - 1) / LG_MIN_WG * LG_MIN_WG, most = (dense ? 2 : 1) * LG_MAX_WG;
     return want < most ? want : most;
 }
 // Instances in a batch above which it runs on dense kernels, where a class has

@@ -1631,9 +1631,12 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     for (int c = 1; c < NG; c++) first[c] = first[c - 1] + count[c - 1];
     // Within a group the expensive instances come first (the gangs take them in
     // order), so the last ones to run are short: a 256-point sweep ends 10 ms
-    // earlier than in the caller's order.  A group's share of the gangs follows
-    // its share of the cost; the last one asks for all of them, and its
-    // workgroups take the CUs that the others leave.
+    // earlier than in the caller's order.  Every group asks for as many gangs as
+    // it has instances, up to the whole chip: those of the groups behind take the
+    // CUs that the ones in front leave.  (Shares of the CUs that followed the
+    // groups' estimated costs left CUs idle where the estimates were off: 40
+    // instances at 16384, 40 with Raman at 8192 and 40 at 4096 20.9 ms, now 10.1;
+    // 60 envelope instances beside 120 at 16384 90 ms, now 13; equal for sweeps.)
     std::vector<int> pos(n), by_cost(n);
     std::vector<double> cost(n);
     for (int i = 0; i < n; i++) {
@@ -1641,29 +1644,23 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         by_cost[i] = i;
     }
     std::stable_sort(by_cost.begin(), by_cost.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    double group_cost[NG] = {0}, all_cost = 0.0;
-    int nwg[NG] = {0}, last_gang = -1, n_gang = 0;
+    int nwg[NG] = {0}, n_dense = 0;
     bool dense[NG] = {false};
+    const auto is_gang = [](int c) { return c < V_ZDEP * LH_NCLASS && c != LH_CLASS_RADIAL; };
+    const auto has_dense = [&](int c) { return is_gang(c) && lg_has_dense(c % LH_NCLASS, c >= V_RAMAN * LH_NCLASS); };
     {
         int fill[NG] = {0};
         for (int i : by_cost) {
             const int c = group_of(ctxs[i]);
             pos[i] = first[c] + fill[c]++;
-            if (c < V_ZDEP * LH_NCLASS && c != LH_CLASS_RADIAL) group_cost[c] += cost[i], all_cost += cost[i];
         }
     }
-    for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
-        if (c != LH_CLASS_RADIAL) n_gang += count[c];
-    for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
-        dense[c] = n_gang > LG_DENSE_ABOVE && lg_has_dense(c % LH_NCLASS, c >= V_RAMAN * LH_NCLASS);
-    for (int gi = 0; gi < NG; gi++) {
-        const int c = (gi % N_VAR) * LH_NCLASS + order[gi / N_VAR];
-        if (!count[c] || c >= V_ZDEP * LH_NCLASS || c == LH_CLASS_RADIAL) continue;
-        const double share = all_cost > 0.0 ? group_cost[c] / all_cost : 1.0;
-        nwg[c] = lg_workgroups(count[c], share, dense[c]);
-        last_gang = c;
+    for (int c = 0; c < NG; c++)
+        if (is_gang(c)) n_dense += count[c];
+    for (int c = 0; c < NG; c++) {
+        dense[c] = has_dense(c) && n_dense > LG_DENSE_ABOVE;
+        if (count[c] && is_gang(c)) nwg[c] = lg_workgroups(count[c], dense[c]);
     }
-    if (last_gang >= 0) nwg[last_gang] = lg_workgroups(count[last_gang], 1.0, dense[last_gang]);
     // one device block: the instances' records, each class's control block, the
     // run counters
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };

@@ -97,3 +97,26 @@ def test_even_batch_against_one(pkg, capi, init_dz):
 
     assert (st[64].steps, st[64].rejected) == (s.steps, s.rejected)
     assert err(states[64], E) <= 1e-6 and err(saves[64], sv) <= 1e-6
+
+
+def test_kinds_of_grid_beside_each_other(pkg, capi):
+    """Field and envelope instances in one batch, whose estimated costs cannot be
+    compared: both on gangs, and together about as long as one after the other."""
+    print("case: 40 envelope instances beside 100 field ones", flush=True)
+    from luna_jl_amd import configs, runtime
+    c = configs.capillary_instance(energy=80e-6, pressure=1.0, trange=1e-12, flength=0.1, ppt_n=2 ** 12)
+    g = configs.gnlse_instance(trange=6e-12, flength=0.005)
+    parts = [(c.holder, c.Ew0, capi.rk_opts(0.05, save_n=2, init_dz=2e-3))] * 100
+    parts += [(g.holder, g.Ew0, capi.rk_opts(0.001, save_n=2, init_dz=1e-4))] * 40
+    ctxs = [runtime.Context(h) for h, _, _ in parts]
+
+    def ms(sel):
+        run = lambda: runtime.batch_solve_opts([ctxs[i] for i in sel], [parts[i][1] for i in sel], [parts[i][2] for i in sel], want_saves=False)
+        run()
+        assert all(s.status == 0 for s in run()[3])
+        return max(t for t, _ in runtime.last_launch_times().values())
+
+    field, env, both = ms(range(100)), ms(range(100, 140)), ms(range(140))
+    print(f"ms: {field:.2f} {env:.2f} {both:.2f}", flush=True)
+    assert runtime.last_launch_kinds() == {16384: capi.LH_KIND_GANG, "env8192": capi.LH_KIND_GANG}
+    assert both <= 2 * (field + env)
