@@ -33,14 +33,15 @@ static inline int lg_workgroups(int n, bool dense) {
     const int want = (LG_G * n + LG_MIN_WG - 1) / LG_MIN_WG * LG_MIN_WG, most = (dense ? 2 : 1) * LG_MAX_WG;
     return want < most ? want : most;
 }
-// Instances in a batch above which it runs on dense kernels, where a class has
-// one.  A gang on half the registers and half a CU per member takes 1.6 times as
-// long for a step, two of them do 1.25 times as much: better once there are two
-// to three instances for each of the 64 gangs, before that the longest instance
-// decides.  ms for n propagations of 0.4 m (half Nto = 8192, half 16384), one
-// workgroup per CU / two: 128 23.2/29.0, 160 27.7/29.7, 192 34.4/30.3, 224
-// 38.8/33.2, 256 44.6/40.0; 384 of 0.2 m 35.3/34.0.
-static constexpr int LG_DENSE_ABOVE = 176;
+// Instances of the classes that have one above which a batch runs on dense
+// kernels.  A gang on half the registers and half a CU per member takes 1.6
+// times as long for a step, two of them do 1.25 times as much: better once 64
+// gangs would take a third round, before that the longest instance decides.  ms,
+// one workgroup per CU / two, energies and pressures at random, Nto = 8192: 96
+// 7.6/8.3, 128 9.2/8.7, 144 11.0/9.2, 160 11.5/10.0, 192 12.8/12.4, 256 16.8/14.8;
+// 16384: 96 10.0/11.7, 128 12.3/12.8, 144 15.2/13.7, 160 16.0/15.0, 192 17.5/17.1,
+// 256 23.0/20.3; both: 128 11.0/12.2, 160 13.9/13.3, 192 15.7/13.9, 256 18.9/17.2.
+static constexpr int LG_DENSE_ABOVE = 128;
 static inline void lg_ctl_init(void* p, int njobs, int nwg, const unsigned* beat) {
     memset(p, 0, lg_ctl_bytes(njobs, nwg));
     GangCtl* c = (GangCtl*)p;

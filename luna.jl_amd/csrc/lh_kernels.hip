@@ -1656,7 +1656,7 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         }
     }
     for (int c = 0; c < NG; c++)
-        if (is_gang(c)) n_dense += count[c];
+        if (has_dense(c)) n_dense += count[c];
     for (int c = 0; c < NG; c++) {
         dense[c] = has_dense(c) && n_dense > LG_DENSE_ABOVE;
         if (count[c] && is_gang(c)) nwg[c] = lg_workgroups(count[c], dense[c]);
