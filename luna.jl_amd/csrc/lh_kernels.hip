@@ -749,9 +749,9 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
 
 // Whether the constant-fill instances of a batch run on one workgroup each
 // (lh_solo_kernel.h) instead of on gangs.  Both ways are priced with the
-// estimated lengths of their runs, dealt longest first to the places there are:
-// 256 workgroups alone, 64 gangs or 128 dense ones; gangs share the chip between
-// classes, which costs a tenth or more of their work.  Equal instances come in
+// estimated lengths of their runs (a run without nonlinear phase still takes a
+// tenth of the longest one's steps), dealt longest first to the places there
+// are: 256 workgroups alone, 64 gangs or 128 dense ones.  Equal instances come in
 // rounds: 65 to 128 of them occupy 64 gangs as long as 128 do.  µs per
 // right-hand side, one workgroup 23.4, 37.4, 63.7 at Nto = 4096, 8192, 16384;
 // gangs, per instance on the whole chip, 0.275, 0.31, 0.455 at one workgroup per
@@ -759,14 +759,18 @@ static double solve_cost(const lh_ctx* c, const lh_rk_opts* o) {
 // likewise (with a Raman response; the envelope grid of 4096 points).  Field
 // grids without an entry, and envelope grids of 8192 points and more, have no
 // kernel for one workgroup: at 16 to 512 equal instances gangs took 0.2 to 0.97
-// of the time that one did when it had.
+// of the time that one did when it had.  The estimates of field grids, of those
+// with a Raman response and of envelope grids cannot be compared, so a batch with
+// more than one of them stays on gangs.
 // Equal instances, ms alone / on gangs: Nto = 4096, 72 3.3/5.9; 8192, 72 5.3/6.5;
 // 16384, 72 9.8/9.7; Raman 4096, 72 12.2/14.7, 8192, 72 21.9/17.9, 176 24.2/28.5;
-// envelope 4096, 72 10.5/9.0, 256 of each field grid 3.8, 6.1, 10.4 against 10.1,
-// 10.9, 16.0.  Sweeps whose longest run is twice the mean: 51 against 40 ms with
-// 256 points, 26 against 34 with 384 (half as long), 53 against 76 with 512.  The
-// rule depends on the batch alone, so a batch gives the same bits every time;
-// what the two ways differ by is with lh_batch_solve in luna_hip.h.
+// envelope 4096, 72 10.5/9.0; 256 of each field grid 3.8, 6.1, 10.4 against 10.1,
+// 10.9, 16.0.  Energies and pressures at random: 8192, 160 10.5/10.0, 176
+// 10.6/11.3, 256 11.1/14.8; 16384, 224 19.4/18.9, 256 20.0/20.3; 4096, 128
+// 6.1/8.4; sweeps over both, 256 20.9/17.2, 300 21.6/20.2, 384 22.1/25.1, 512
+// 24.0/31.9: the rule takes the faster way in each.  It depends on the batch
+// alone, so a batch gives the same bits every time; what the two ways differ by
+// is with lh_batch_solve in luna_hip.h.
 struct SoloPrice {
     double alone, gang, dense;  // µs: alone per right-hand side, on gangs per instance
 };
@@ -805,22 +809,29 @@ static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
     std::vector<double> cost;
     std::vector<SoloPrice> price;
     SoloPrice p;
-    for (int i = 0; i < n; i++)
-        if (solo_price(ctxs[i], &p)) {
-            cost.push_back(solve_cost(ctxs[i], op[i]) / class_us(ctx_class(ctxs[i])));
-            price.push_back(p);
-        }
-    if (cost.empty()) return false;
-    if (*std::max_element(cost.begin(), cost.end()) == 0.0) cost.assign(cost.size(), 1.0);  // linear runs: equal lengths
+    bool kind[3] = {false, false, false};
+    int n_dense = 0;
+    for (int i = 0; i < n; i++) {
+        const lh_desc& d = ctxs[i]->d;
+        if (d.transform == LH_TRANS_MODEAVG && !ctxs[i]->zg_on) kind[d.grid_kind == LH_GRID_ENV ? 2 : field_raman(d) ? 1 : 0] = true;
+        if (!solo_price(ctxs[i], &p)) continue;
+        cost.push_back(solve_cost(ctxs[i], op[i]) / class_us(ctx_class(ctxs[i])));
+        price.push_back(p);
+        n_dense += p.dense > 0;
+    }
+    if (cost.empty() || kind[0] + kind[1] + kind[2] > 1) return false;
+    const double longest = *std::max_element(cost.begin(), cost.end());
     std::vector<double> alone, gang, dense;
     double work = 0.0;
     for (size_t i = 0; i < cost.size(); i++) {
-        const bool d = n > LG_DENSE_ABOVE && price[i].dense > 0;
-        alone.push_back(cost[i] * price[i].alone);
-        (d ? dense : gang).push_back(cost[i] * (d ? 2 * GANGS * price[i].dense : GANGS * price[i].gang));
-        work += cost[i] * (d ? price[i].dense : price[i].gang);
+        const double c = longest > 0.0 ? cost[i] + 0.1 * longest : 1.0;  // linear runs: equal lengths
+        const bool d = n_dense > LG_DENSE_ABOVE && price[i].dense > 0;
+        alone.push_back(c * price[i].alone);
+        (d ? dense : gang).push_back(c * (d ? 2 * GANGS * price[i].dense : GANGS * price[i].gang));
+        work += c * (d ? price[i].dense : price[i].gang);
     }
-    return dealt(alone, LG_MAX_WG) < std::max({1.1 * work, dealt(gang, GANGS), dealt(dense, 2 * GANGS)});
+    // the gangs' tails and the estimates' errors: a tenth of the work, 7 % of the dealing
+    return dealt(alone, LG_MAX_WG) < std::max(1.1 * work, 1.07 * std::max(dealt(gang, GANGS), dealt(dense, 2 * GANGS)));
 }
 
 static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, bool alone, DInst* in,

@@ -120,3 +120,17 @@ def test_kinds_of_grid_beside_each_other(pkg, capi):
     print(f"ms: {field:.2f} {env:.2f} {both:.2f}", flush=True)
     assert runtime.last_launch_kinds() == {16384: capi.LH_KIND_GANG, "env8192": capi.LH_KIND_GANG}
     assert both <= 2 * (field + env)
+
+
+def test_kinds_that_cannot_be_compared(pkg, capi):
+    """Even instances go to one workgroup each only where all of the batch are of
+    one kind: with a Raman gas or an envelope grid beside them they stay on gangs."""
+    print("case: even instances beside others", flush=True)
+    from luna_jl_amd import configs
+    c = configs.capillary_instance(energy=80e-6, pressure=1.0, trange=0.25e-12, flength=0.1, ppt_n=2 ** 12)
+    opts = capi.rk_opts(1e-3, save_n=2, init_dz=1e-3)
+    assert kinds_of([c.holder] * 100, [c.Ew0] * 100, opts) == {4096: capi.LH_KIND_ALONE}
+    raman, env = test_gpu_solo_kinds._molecular(0.25e-12), test_gpu_solo_kinds._envelope()
+    assert kinds_of([c.holder] * 100 + [raman[0]], [c.Ew0] * 100 + [raman[1]], opts) == {4096: capi.LH_KIND_GANG}
+    k = kinds_of([c.holder] * 100 + [env[0]], [c.Ew0] * 100 + [env[1]], opts)
+    assert k == {4096: capi.LH_KIND_GANG, "env4096": capi.LH_KIND_GANG}
