@@ -13,6 +13,14 @@
 // --------------------------------------------------------------------------
 // Device-side instance description
 // --------------------------------------------------------------------------
+// An instance's counters, and a word that any workgroup sets which lost another
+// one of its gang (lh_gang_proto.h): the run's status is then LH_E_HIP, whatever
+// the one that wrote the counters knew.
+struct RunStats {
+    lh_stats s;
+    int lost, pad;
+};
+
 struct DInst {
     int grid_kind, transform, n_omega, n_t, n_to, n_r;
     int kerr, plasma, raman, ppt_n;
@@ -38,7 +46,7 @@ struct DInst {
     long long kstride;
     double2* saves;       // [save_n][n_state] or null
     const double* zgrid;  // [save_n]
-    lh_stats* stats;
+    RunStats* stats;
     double z0, zmax, rtol, atol, safety, max_dz, min_dz, init_dz;
     int repeat_limit, save_n;
     int save_first;       // saves already written (a resumed run continues at this index)
@@ -1044,7 +1052,7 @@ enum {
     LH_CLASS_ENV8192 = 3,  // envelope grid, Nto = Nt = 8192
     LH_CLASS_ENV4096 = 4,  // envelope grid, Nto = Nt = 4096
     LH_CLASS_RADIAL = 5,   // radial transform (solved context by context)
-    LH_CLASS_ENV16384 = 6, // envelope grid, Nto = Nt = 16384, transforms staged through HBM
-    LH_CLASS_32768 = 7,    // field grid, Nto = 32768, Nt = 16384, transforms staged through HBM
+    LH_CLASS_ENV16384 = 6, // envelope grid, Nto = Nt = 16384
+    LH_CLASS_32768 = 7,    // field grid, Nto = 32768, Nt = 16384
     LH_NCLASS = 8
 };

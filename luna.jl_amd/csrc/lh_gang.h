@@ -20,8 +20,8 @@
 // right-hand side with plasma has four, whatever the gang's size, so the gain
 // per added CU falls: four members are a compromise between one propagation
 // alone and a sweep that fills the chip.  Measured against one workgroup per
-// instance (one MI355X): a propagation at Nto = 8192 18.4 → 11.1 ms, envelope
-// Nt = 8192 with Raman 274 → 89 ms, Nt = 16384 57.4 → 12.1 ms, a single
+// instance (one MI355X): a propagation at Nto = 8192 18.4 → 10.6 ms, envelope
+// Nt = 8192 with Raman 274 → 87 ms, Nt = 16384 57.4 → 11.8 ms, a single
 // right-hand side at Nto = 16384 56 → 38 us; a 64-point sweep 41.6 → 19.6 ms,
 // 256 points 47.1 → 45.2 ms.
 //
@@ -1526,8 +1526,9 @@ __device__ __forceinline__ void g_solve(const DInst& in, SM& sm, Gang& g) {
         __syncthreads();
     }
     for (int p = fresh_tid(); p < nb; p += LH_T) gl(in.Y)[Z::k_of(h, p)] = gl(Y)[p];
-    gang_sync(g, sm);  // whoever lost a member says so before the record is written
-    if (sm.gflag == LG_LOST) status = LH_E_HIP;
+    // (a word of its own: agreeing on the status at one more barrier, with the
+    // counters in registers, cost a dense kernel 10 spills and a sweep 1.5 %)
+    if (sm.gflag == LG_LOST && threadIdx.x == 0) lg_st(&in.stats->lost, 1);
     if (h == 0 && threadIdx.x == 0 && gl(in.stats)) {
         lh_stats s;
         s.steps = steps;
@@ -1538,7 +1539,7 @@ __device__ __forceinline__ void g_solve(const DInst& in, SM& sm, Gang& g) {
         s.saved = saved;
         s.z = tn;
         s.dz = dtn;
-        *in.stats = s;
+        in.stats->s = s;
     }
     __syncthreads();
 }
@@ -1614,7 +1615,7 @@ __device__ __forceinline__ void gang_area(Gang& g, const DInst& in) {
     g.P = g.rec + 512;
 }
 
-// DENSE: compiled for two workgroups per CU (128 registers; 115 of the field
+// DENSE: compiled for two workgroups per CU (128 registers; 128 of the field
 // kernel's values at Nto = 16384 spill, most of them around the transform
 // passes; 204 with three bins per thread in a round of loads).  The same source,
 // so the same bits; the loads of a round alone are grouped differently.

@@ -2,7 +2,7 @@
 // batches, streaming, plans; and the kernels that are not in lh_gang.h.
 //
 // Mode-averaged instances run on gangs of four workgroups (lh_gang.h), those
-// with a z-dependent fill on one workgroup (lh_solo.hip), radial ones as a
+// with a z-dependent fill on one workgroup (lh_solo_kernel.h), radial ones as a
 // launch sequence (lh_radial.hip).  A right-hand side keeps its time series in
 // LDS:
 //   stage prologue (ȳ = y + Δz Σ B k, ·exp(LΔ)) → c2r pre-pack → inverse
@@ -186,7 +186,7 @@ struct lh_ctx {
     int zgrid_cap;
     double* zgrid_h;  // host copy of the save grid in zgrid (an unchanged grid is not uploaded again)
     int zgrid_hn;
-    lh_stats* dstats;
+    RunStats* dstats;
     unsigned char* launch1;  // one instance's solve: control block, then its DInst
     unsigned* beat;          // the device's
     RhsSet rset[RHS_SETS];
@@ -537,7 +537,7 @@ static DInst base_inst(const lh_ctx* c) {
         in.zfdt = c->zfdt;
         in.zL = c->zL;
         in.zOF = c->zOF;
-        in.linop = c->zL;  // refreshed in place at every new z (lh_solo.hip)
+        in.linop = c->zL;  // refreshed in place at every new z (lh_solo_kernel.h)
         in.outfac = c->zOF;
     }
     return in;
@@ -545,8 +545,13 @@ static DInst base_inst(const lh_ctx* c) {
 
 // The counters of an instance until its solver writes them: what a launch whose
 // gangs never form leaves.
-__host__ __device__ static lh_stats unsolved(const DInst& in) {
-    return lh_stats{0, 0, 0, 0, LH_E_HIP, in.save_first, in.z0, in.init_dz};
+__host__ __device__ static RunStats unsolved(const DInst& in) {
+    return RunStats{{0, 0, 0, 0, LH_E_HIP, in.save_first, in.z0, in.init_dz}, 0, 0};
+}
+static lh_stats solved(const RunStats& r) {
+    lh_stats s = r.s;
+    if (r.lost) s.status = LH_E_HIP;
+    return s;
 }
 
 // A launch over one instance: its control block, then its DInst.  A kernel that
@@ -835,7 +840,7 @@ static bool solo_pays(lh_ctx* const* ctxs, const lh_rk_opts* const* op, int n) {
 }
 
 static int prepare_instance(lh_ctx* c, const lh_rk_opts* o, bool want_saves, bool alone, DInst* in,
-                            lh_stats* dstats_slot, hipStream_t s) {
+                            RunStats* dstats_slot, hipStream_t s) {
     if (!opts_ok(o)) return LH_E_ARG;
     if (!c->have_state) return LH_E_ARG;
     int st = ensure_solver_buffers(c, o->save_n, want_saves, alone);
@@ -1246,7 +1251,7 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
     if (!st && modeavg &&
         (hipEventCreateWithFlags(&c->cap_ev, hipEventDisableTiming) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess))
         st = LH_E_HIP;
-    if (!st && hipMalloc(&c->dstats, sizeof(lh_stats)) != hipSuccess) st = LH_E_NOMEM;
+    if (!st && hipMalloc(&c->dstats, sizeof(RunStats)) != hipSuccess) st = LH_E_NOMEM;
     if (st) {
         lh_destroy(c);
         return st;
@@ -1525,7 +1530,9 @@ int lh_solve_stream(lh_ctx* c, double* Ew, const lh_rk_opts* o, lh_output_cb cb,
         nanosleep(&ts, nullptr);
     }
     if (!st) {
-        if (hipMemcpy(stats, c->dstats, sizeof(lh_stats), hipMemcpyDeviceToHost) != hipSuccess) st = LH_E_HIP;
+        RunStats rs;
+        if (hipMemcpy(&rs, c->dstats, sizeof(rs), hipMemcpyDeviceToHost) != hipSuccess) st = LH_E_HIP;
+        if (!st) *stats = solved(rs);
         if (!st && lapped) stats->status = LH_E_HOST_WAIT;
     } else {
         (void)hipStreamSynchronize(c->stream);  // never free a block the kernel may still write
@@ -1681,11 +1688,11 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
         if (count[c] && c < V_ZDEP * LH_NCLASS && c != LH_CLASS_RADIAL)
             total += up(lg_ctl_bytes(count[c], nwg[c]));
     }
-    const size_t st_off = total, in_bytes = st_off + sizeof(lh_stats) * (size_t)n;
+    const size_t st_off = total, in_bytes = st_off + sizeof(RunStats) * (size_t)n;
     unsigned char* dblk = nullptr;
     HIPCK(hipMalloc(&dblk, in_bytes));
     const DInst* dinst = (const DInst*)dblk;
-    lh_stats* dstats = (lh_stats*)(dblk + st_off);
+    RunStats* dstats = (RunStats*)(dblk + st_off);
     std::vector<unsigned char> hblk(in_bytes);
     DInst* h = (DInst*)hblk.data();
     for (int c = 0; c < V_ZDEP * LH_NCLASS; c++)
@@ -1693,7 +1700,7 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     for (int i = 0; i < n && !st; i++)
         st = prepare_instance(ctxs[i], op[i], want_saves != 0, pos[i] >= first[V_ZDEP * LH_NCLASS], &h[pos[i]],
                               dstats + pos[i], s0);
-    for (int i = 0; i < n && !st; i++) ((lh_stats*)(hblk.data() + st_off))[i] = unsolved(h[i]);
+    for (int i = 0; i < n && !st; i++) ((RunStats*)(hblk.data() + st_off))[i] = unsolved(h[i]);
     if (!st && hipMemcpyAsync(dblk, hblk.data(), in_bytes, hipMemcpyHostToDevice, s0) != hipSuccess) st = LH_E_HIP;
     std::vector<lh_stats> rad_stats(n);
     hipEvent_t ready = nullptr, done[NG] = {nullptr}, t0[NG] = {nullptr}, t1[NG] = {nullptr};
@@ -1727,8 +1734,8 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
             hipEventRecord(done[c], cs) != hipSuccess || hipStreamWaitEvent(s0, done[c], 0) != hipSuccess)
             st = st ? st : LH_E_HIP;
     }
-    std::vector<lh_stats> hs(n);
-    if (!st && hipMemcpyAsync(hs.data(), dstats, sizeof(lh_stats) * (size_t)n, hipMemcpyDeviceToHost, s0) != hipSuccess)
+    std::vector<RunStats> hs(n);
+    if (!st && hipMemcpyAsync(hs.data(), dstats, sizeof(RunStats) * (size_t)n, hipMemcpyDeviceToHost, s0) != hipSuccess)
         st = LH_E_HIP;
     if (hipStreamSynchronize(s0) != hipSuccess && !st) st = LH_E_HIP;
     float cls_ms[LH_NCLASS] = {0};
@@ -1756,7 +1763,7 @@ static int batch_resident(lh_ctx* const* ctxs, int n, const lh_rk_opts* const* o
     (void)hipFree(dblk);
     if (st) return st;
     for (int i = 0; i < n; i++) {
-        stats[i] = (ctx_class(ctxs[i]) == LH_CLASS_RADIAL) ? rad_stats[i] : hs[pos[i]];
+        stats[i] = (ctx_class(ctxs[i]) == LH_CLASS_RADIAL) ? rad_stats[i] : solved(hs[pos[i]]);
         ctxs[i]->last_status = stats[i].status;
         ctxs[i]->have_result = 1;
         ctxs[i]->result_nrec = ctxs[i]->st_on ? (int)(stats[i].accepted < ctxs[i]->st_cap ? stats[i].accepted : ctxs[i]->st_cap) : 0;
@@ -2194,15 +2201,17 @@ static NoallocLayout noalloc_layout(const lh_desc& d, int save_n) {
     NoallocLayout L;
     L.inst = 0;
     L.stats = up(LAUNCH1_BYTES);
-    L.zgrid = L.stats + up(sizeof(lh_stats));
+    L.zgrid = L.stats + up(sizeof(RunStats));
     L.k = L.zgrid + up(sizeof(double) * (size_t)(save_n > 0 ? save_n : 1));
     L.total = L.k + sizeof(double2) * lg_stride(d) * LG_SLOTS;
     return L;
 }
 
-// The problems lh_solve_noalloc takes: record (1 KB), counters, save grid, a second
-// state, eight stage vectors and the envelope Raman or staged-transform series
-// within LH_NOALLOC_SCRATCH_BYTES.
+// The problems lh_solve_noalloc takes.  The bound is what a solver with one
+// workgroup needs: record (1 KB), counters, save grid, a second state, eight
+// stage vectors and the series of a Raman response or of the largest grids within
+// LH_NOALLOC_SCRATCH_BYTES; the gangs' layout (noalloc_layout) of every such
+// problem fits the array.
 static bool noalloc_fits(const lh_ctx* c, int save_n) {
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const lh_desc& d = c->d;
@@ -2238,7 +2247,7 @@ int lh_solve_noalloc(lh_ctx* c, void* Ew_dev, const lh_rk_opts* o, void* saves_d
     in.kstride = (long long)lg_stride(c->d);
     in.saves = (double2*)saves_dev;
     in.zgrid = (const double*)(base + L.zgrid);
-    in.stats = (lh_stats*)(base + L.stats);
+    in.stats = (RunStats*)(base + L.stats);
     inst_options(&in, o);
     // Nothing in the working memory needs clearing: the kernel writes every
     // state and stage vector before reading it, and the counters at the end.
@@ -2261,9 +2270,10 @@ int lh_solve_noalloc(lh_ctx* c, void* Ew_dev, const lh_rk_opts* o, void* saves_d
     else if (!launch_solve(l, c->d.raman != 0, false))
         return LH_E_ARG;
     HIPCK(hipGetLastError());
-    lh_stats hs;
-    HIPCK(hipMemcpyAsync(&hs, base + L.stats, sizeof(lh_stats), hipMemcpyDeviceToHost, s));
+    RunStats rs;
+    HIPCK(hipMemcpyAsync(&rs, base + L.stats, sizeof(rs), hipMemcpyDeviceToHost, s));
     HIPCK(hipStreamSynchronize(s));
+    const lh_stats hs = solved(rs);
     if (zsaves && o->save_n > 0) save_grid_into(o, zsaves);
     *stats = hs;
     c->last_status = hs.status;

@@ -584,7 +584,7 @@ __global__ __launch_bounds__(64) void rad_set(RadArgs a, RadCtl h, RadArgs* ap) 
 // default plan's, halved while the grid leaves half the CUs without a workgroup
 // (a wave with more tiles loads less per product).  Same products in the same
 // order, so the same bits.  A plan from the wisdom or lh_set_plan runs as it is.
-// µs per GEMM with 2 tiles / 1, workgroups at 2 tiles: Nto × Nr = 2048 × 64 (32)
+// µs per GEMM in the kernel trace with 2 tiles / 1, workgroups at 2 tiles: Nto × Nr = 2048 × 64 (32)
 // 6.4/4.5, 4096 × 64 (64) 7.3/5.6, 2048 × 128 (64) 9.5/7.4, 8192 × 64 (128)
 // 7.6/6.0, 2048 × 256 (128) 15.7/12.2; 4096 × 192 (192) 13.9/15.3, 8192 × 128
 // (256) 10.2/11.7, 8192 × 256 (512) 28.1/31.6.

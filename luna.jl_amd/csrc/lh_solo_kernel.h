@@ -965,7 +965,7 @@ __device__ __forceinline__ void solo_solve(const DInst& in, Smem& sm) {
         s.saved = saved;
         s.z = tn;
         s.dz = dtn;
-        *in.stats = s;
+        in.stats->s = s;
     }
     __syncthreads();
 }

@@ -72,14 +72,14 @@ struct Launch {
     std::vector<unsigned long long> block;
     GangCtl* ctl;
     std::vector<std::vector<long>> x;  // [job][member]: the series
-    std::vector<int> status, wrong, runs;
+    std::vector<int> status, lost_in, wrong, runs;
     int launch_status = -1;
     unsigned beat = 0;
     std::atomic<int> lost{0};          // members that count another one as lost
     std::function<void(int, int, int)> wait = [](int, int, int) {};
     std::function<void(int)> arrive = [](int) {};  // before workgroup i takes a ticket
     Launch(int njobs, int nwg) : block(lg_ctl_bytes(njobs, nwg) / 8 + 1), x(njobs, std::vector<long>(LG_G)),
-                                 status(njobs, LG_LOST), wrong(njobs), runs(njobs) {
+                                 status(njobs, LG_LOST), lost_in(njobs), wrong(njobs), runs(njobs) {
         ctl = (GangCtl*)block.data();
         ctl->njobs = njobs;
         ctl->n_wg = nwg;
@@ -123,7 +123,7 @@ struct Launch {
                 }
                 __atomic_fetch_add(&beat, 1, __ATOMIC_SEQ_CST);
             }
-            sync(flags, h, ep, flag, gflag);
+            if (gflag == LG_LOST) __atomic_store_n(&lost_in[job], 1, __ATOMIC_SEQ_CST);
             if (h == 0) status[job] = gflag;
         }
         if (ctl->njobs == 1) {
@@ -135,6 +135,8 @@ struct Launch {
         std::vector<std::thread> th;
         for (size_t i = 0; i < xcc.size(); i++) th.emplace_back([this, i, &xcc] { group((int)i, xcc[i]); });
         for (auto& t : th) t.join();
+        for (size_t j = 0; j < status.size(); j++)
+            if (lost_in[j]) status[j] = LG_LOST;
     }
 };
 static std::vector<int> spread(int nwg, int nx) {
