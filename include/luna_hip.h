@@ -31,7 +31,9 @@ extern "C" {
 enum {
     LH_OK = 0,
     LH_E_ARG = 1,          /* invalid argument / unsupported size            */
-    LH_E_HIP = 2,          /* HIP runtime error                              */
+    LH_E_HIP = 2,          /* HIP runtime error; of a run: the four workgroups
+                              that share it did not come together (a stream
+                              with fewer than four CUs per XCD)              */
     LH_E_PPT_RANGE = 3,    /* |E| above the PPT table maximum                */
     LH_E_REPEAT_LIMIT = 4, /* more than repeat_limit consecutive rejections  */
     LH_E_NONFINITE = 5,    /* non-finite state                               */

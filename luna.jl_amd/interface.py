@@ -68,7 +68,7 @@ def run(Ew, grid, linop, transform, FT=None, output=None, min_dz=0.0, max_dz=Non
         try:
             ctx.set_step_stats(statsfun)
         except _capi.LunaHipError as e:
-            # the grids staged through HBM record no statistics on the device
+            # the largest grids record no statistics on the device
             if e.status != _capi.LH_E_ARG or zdep:
                 raise
             ctx.set_step_stats(None)

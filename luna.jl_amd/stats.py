@@ -153,8 +153,8 @@ class StatsFun:
 
     def host_record(self, Ew, z, dz):
         """The record the propagation kernel writes (the same values and
-        formulas), evaluated on the host: for the grids whose transforms are
-        staged through HBM, where the kernel records no statistics."""
+        formulas), evaluated on the host: for the largest grids (envelope
+        Nt = 16384, field Nto = 32768), where the kernel records none."""
         K = _capi.STAT_KEYS.index
         g = self.grid
         Ew = np.asarray(Ew).reshape(-1)
