@@ -590,14 +590,28 @@ static constexpr size_t RHS_STATUS = LAUNCH1_CTL, RHS_GX = LAUNCH1_CTL + 256;
 __global__ __launch_bounds__(64) void lh_clear_ctl(unsigned* ctl, const unsigned* beat) {
     lg_ctl_clear(ctl, LAUNCH1_CTL, beat);
 }
+static size_t rhs_block_bytes(const lh_ctx* c) {
+    return RHS_GX + sizeof(double2) * (lg_area_len(c->d) + (field_raman(c->d) ? (size_t)c->d.n_to : 0));
+}
 // Makes a set ready for launches on s (ordered on s; allocates what is missing).
 static int rhs_set_ready(lh_ctx* c, RhsSet* r, hipStream_t s) {
     if (!r->block) {
-        HIPCK(hipMalloc(&r->block, RHS_GX + sizeof(double2) * (lg_area_len(c->d) + (field_raman(c->d) ? (size_t)c->d.n_to : 0))));
+        HIPCK(hipMalloc(&r->block, rhs_block_bytes(c)));
         hipLaunchKernelGGL(lh_clear_ctl, dim3(1), dim3(64), 0, s, (unsigned*)r->block, c->beat);
         HIPCK(hipGetLastError());
     }
     if (c->zg_on && !r->z) HIPCK(hipMalloc(&r->z, sizeof(double2) * 2 * lg_stride(c->d)));
+    return LH_OK;
+}
+// The first two sets.  Their control blocks are copied: a kernel would bind the
+// context's stream to a hardware queue, which takes a millisecond.
+static int rhs_sets_init(lh_ctx* c) {
+    alignas(256) unsigned char h[RHS_GX] = {};
+    lg_ctl_init(h, 1, LG_MIN_WG, c->beat);
+    for (const int i : {RHS_FIRST, RHS_CAPTURED}) {
+        if (hipMalloc(&c->rset[i].block, rhs_block_bytes(c)) != hipSuccess) return LH_E_NOMEM;
+        HIPCK(hipMemcpy(c->rset[i].block, h, sizeof(h), hipMemcpyHostToDevice));
+    }
     return LH_OK;
 }
 
@@ -611,6 +625,7 @@ static int rhs_set_of(lh_ctx* c, hipStream_t s, RhsSet** out) {
         HIPCK(hipStreamGetCaptureInfo(s, &cs, &id));
         if (cs != hipStreamCaptureStatusNone) {
             if (c->cap_stream && c->cap_id == id && c->cap_stream != s) {
+                if (!c->cap_ev) HIPCK(hipEventCreateWithFlags(&c->cap_ev, hipEventDisableTiming));
                 HIPCK(hipEventRecord(c->cap_ev, c->cap_stream));
                 HIPCK(hipStreamWaitEvent(s, c->cap_ev, 0));
             }
@@ -1246,11 +1261,7 @@ int lh_create(lh_ctx** out, const lh_desc* d) {
         st = modeavg ? gang_twiddles(c->device, &tw) : twiddles(c->device, &tw);
     }
     if (!st && modeavg && hipMalloc(&c->launch1, LAUNCH1_BYTES) != hipSuccess) st = LH_E_NOMEM;
-    if (!st && modeavg) st = rhs_set_ready(c, &c->rset[RHS_FIRST], c->stream);
-    if (!st && modeavg) st = rhs_set_ready(c, &c->rset[RHS_CAPTURED], c->stream);
-    if (!st && modeavg &&
-        (hipEventCreateWithFlags(&c->cap_ev, hipEventDisableTiming) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess))
-        st = LH_E_HIP;
+    if (!st && modeavg) st = rhs_sets_init(c);
     if (!st && hipMalloc(&c->dstats, sizeof(RunStats)) != hipSuccess) st = LH_E_NOMEM;
     if (st) {
         lh_destroy(c);
